@@ -74,6 +74,7 @@ _H = C.POINTER(CtrHelicalGeom)
 _SIGS = {
     "ctr_last_error": (C.c_char_p, []),
     "ctr_version": (C.c_int, []),
+    "ctr_release_workspace": (C.c_int, []),
     "ctr_device_info": (C.c_int, [_I, _I, _I, C.c_char_p, C.c_int]),
     "ctr_fan_tables": (C.c_int, [_G, _P, _P, _P]),
     "ctr_fan_angle_tables": (C.c_int, [_G, _P, _P, _P, _P]),

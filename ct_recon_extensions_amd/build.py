@@ -33,7 +33,7 @@ DEVICE_FLAGS = [
     "-munsafe-fp-atomics", "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 
-CORE_SOURCES = ["tables.cpp", "capi.cpp", "classes.cpp", "fan_bp.hip", "par_bp.hip",
+CORE_SOURCES = ["tables.cpp", "workspace.cpp", "capi.cpp", "classes.cpp", "fan_bp.hip", "par_bp.hip",
                 "fp_par.hip", "filter.hip", "ragged.hip", "toeplitz.hip", "par_svbp.hip",
                 "fp_rc.hip", "fp_dd.hip", "helical.hip"]
 NUMPY_SOURCES = ["npext.cpp"]

@@ -503,7 +503,7 @@ int launch_bp_gather_t(const typename Geo::Problem& P, const typename Geo::Table
     const size_t bytes = gather_workspace_bytes<Anchor>(P.na, P.nx, P.ny, nbatch);
     void* own = nullptr;
     if (!ws) {
-        CTR_HIP(hipMallocAsync(&own, bytes, st));
+        CTR_HIP(ctr::ws_alloc(&own, bytes, st));
         ws = own;
     }
     auto* table = static_cast<Anchor*>(ws);
@@ -532,7 +532,7 @@ int launch_bp_gather_t(const typename Geo::Problem& P, const typename Geo::Table
         else
             rc = launch_gather_nb<Geo, 1, 4, 128>(L, st);
     }
-    if (own) CTR_HIP(hipFreeAsync(own, st));
+    if (own) CTR_HIP(ctr::ws_free(own, st));
     return rc;
 }
 

@@ -134,13 +134,13 @@ struct DevTemp {
     explicit DevTemp(hipStream_t s) : st(s) {}
     ~DevTemp()
     {
-        if (p) (void)hipFreeAsync(p, st);
+        if (p) (void)ctr::ws_free(p, st);
     }
     template <typename V>
     bool put(const std::vector<V>& v)
     {
-        if (hipMallocAsync(&p, v.size() * sizeof(V), st) != hipSuccess) {
-            ctr::set_error("hipMallocAsync failed");
+        if (ctr::ws_alloc(reinterpret_cast<void**>(&p), v.size() * sizeof(V), st) != hipSuccess) {
+            ctr::set_error("stream-ordered allocation failed");
             return false;
         }
         return to_device(p, v, st);

@@ -52,6 +52,10 @@ inline double cent_x(const ctr_geom& g) { return static_cast<double>(g.nx - 1) /
 inline double cent_y(const ctr_geom& g) { return static_cast<double>(g.ny - 1) / 2 + g.offset_y; }
 inline double cent_s(const ctr_geom& g) { return static_cast<double>(g.ns - 1) / 2 + g.offset_s; }
 
+// Device memory for the duration of a call, ordered on `st` (workspace.cpp).
+hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st);
+hipError_t ws_free(void* p, hipStream_t st);
+
 // Scale of bp_fan_2d: |orbit| / round(|na*orbit|/pi) (src/bp_fan_2d.cc:58,83).
 double fan_bp_scale(const ctr_geom& g);
 

@@ -131,7 +131,7 @@ int ramp_typed(const ctr_geom& g, const T* in, T* out, unsigned int nrow, const 
     CTR_REQUIRE(lds <= 160 * 1024, CTR_ERR_SHAPE, "ramp filter: ns too large for LDS");
     const int ntaps = 2 * g.ns + 1;
     Acc* hf = nullptr;
-    CTR_HIP(hipMallocAsync(reinterpret_cast<void**>(&hf), ntaps * sizeof(Acc), st));
+    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&hf), ntaps * sizeof(Acc), st));
     hipLaunchKernelGGL(taps_kernel<Acc>, dim3(div_up(ntaps, 256)), dim3(256), 0, st, filter, hf,
                        ntaps);
     int rc = check_launch("taps_kernel");
@@ -145,7 +145,7 @@ int ramp_typed(const ctr_geom& g, const T* in, T* out, unsigned int nrow, const 
                            static_cast<const Acc*>(hf), filter, P);
         rc = check_launch("ramp_kernel");
     }
-    CTR_HIP(hipFreeAsync(hf, st));
+    CTR_HIP(ctr::ws_free(hf, st));
     return rc;
 }
 

@@ -239,7 +239,7 @@ int fp_dd_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const doub
                       static_cast<int>(g.ny), nbatch, g.dx, g.dy};
     T* imgT = nullptr;
     const size_t n = static_cast<size_t>(nbatch) * g.nx * g.ny;
-    CTR_HIP(hipMallocAsync(reinterpret_cast<void**>(&imgT), n * sizeof(T), st));
+    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&imgT), n * sizeof(T), st));
     hipLaunchKernelGGL(dd_transpose_kernel<T>, dim3(div_up(g.nx, 32), div_up(g.ny, 32), nbatch),
                        dim3(32, 8), 0, st, img, imgT, static_cast<int>(g.ny),
                        static_cast<int>(g.nx));
@@ -248,7 +248,7 @@ int fp_dd_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const doub
         rc = nbatch >= 4 ? launch_fp_dd<T, 4>(P, img, imgT, proj, sc, bo, usex, st)
              : nbatch >= 2 ? launch_fp_dd<T, 2>(P, img, imgT, proj, sc, bo, usex, st)
                            : launch_fp_dd<T, 1>(P, img, imgT, proj, sc, bo, usex, st);
-    CTR_HIP(hipFreeAsync(imgT, st));
+    CTR_HIP(ctr::ws_free(imgT, st));
     return rc;
 }
 

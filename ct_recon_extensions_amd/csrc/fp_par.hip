@@ -549,7 +549,7 @@ int fp_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const double*
                 static_cast<int>(g.ny), nbatch, g.dx, g.dy};
     T* imgT = nullptr;
     const size_t n = static_cast<size_t>(nbatch) * g.nx * g.ny;
-    CTR_HIP(hipMallocAsync(reinterpret_cast<void**>(&imgT), n * sizeof(T), st));
+    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&imgT), n * sizeof(T), st));
     hipLaunchKernelGGL(transpose_kernel<T>, dim3(div_up(g.nx, 32), div_up(g.ny, 32), nbatch),
                        dim3(32, 8), 0, st, img, imgT, static_cast<int>(g.ny),
                        static_cast<int>(g.nx));
@@ -561,7 +561,7 @@ int fp_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const double*
             rc = nb == kFpSlices ? launch_fp_lds_v<kFpSlices>(views, P, img, imgT, proj, sc, bo, usex, st)
                  : nb == 2       ? launch_fp_lds_v<2>(views, P, img, imgT, proj, sc, bo, usex, st)
                                  : launch_fp_lds_v<1>(views, P, img, imgT, proj, sc, bo, usex, st);
-            CTR_HIP(hipFreeAsync(imgT, st));
+            CTR_HIP(ctr::ws_free(imgT, st));
             return rc;
         }
     }
@@ -574,7 +574,7 @@ int fp_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const double*
             default: rc = launch_fp<T, 8>(P, img, imgT, proj, sc, bo, usex, st); break;
         }
     }
-    CTR_HIP(hipFreeAsync(imgT, st));
+    CTR_HIP(ctr::ws_free(imgT, st));
     return rc;
 }
 
@@ -607,7 +607,7 @@ int launch_fpt_border(const FpProblem& P, const float* proj, float* img, const d
     const int nchunks = div_up(P.na, cviews);
     double* partial = static_cast<double*>(ws);
     if (!ws)
-        CTR_HIP(hipMallocAsync(reinterpret_cast<void**>(&partial),
+        CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&partial),
                                fpt_border_bytes(P.nx, P.ny, P.na, P.nbatch, cviews), st));
     hipLaunchKernelGGL((fpt_border_partial_kernel<NB>),
                        dim3(div_up(nborder, 256), nchunks, div_up(P.nbatch, NB)), dim3(256), 0, st,
@@ -618,7 +618,7 @@ int launch_fpt_border(const FpProblem& P, const float* proj, float* img, const d
                            dim3(256), 0, st, partial, img, P, nborder, nchunks);
         rc = check_launch("fpt_border_reduce_kernel");
     }
-    if (!ws) CTR_HIP(hipFreeAsync(partial, st));
+    if (!ws) CTR_HIP(ctr::ws_free(partial, st));
     return rc;
 }
 

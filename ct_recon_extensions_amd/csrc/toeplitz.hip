@@ -1060,7 +1060,7 @@ int ramp_toeplitz(const ctr_geom& g, const float* in, float* out, unsigned int n
     const size_t fbytes = ((3 * static_cast<size_t>(ns) + 1) * sizeof(float) + 15) & ~static_cast<size_t>(15);
     const size_t cbytes = bf16x3 ? static_cast<size_t>(2 * nc) * nrev * sizeof(__bf16) : 0;
     unsigned char* scratch = nullptr;
-    CTR_HIP(hipMallocAsync(reinterpret_cast<void**>(&scratch), fbytes + cbytes, st));
+    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&scratch), fbytes + cbytes, st));
     float* hf = reinterpret_cast<float*>(scratch);
     float* w = weight_type ? hf + 2 * ns + 1 : nullptr;
     __bf16* copies = bf16x3 ? reinterpret_cast<__bf16*>(scratch + fbytes) : nullptr;
@@ -1112,7 +1112,7 @@ int ramp_toeplitz(const ctr_geom& g, const float* in, float* out, unsigned int n
         hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, P);
         rc = check_launch("ramp_mfma_kernel");
     }
-    CTR_HIP(hipFreeAsync(scratch, st));
+    CTR_HIP(ctr::ws_free(scratch, st));
     return rc;
 }
 
