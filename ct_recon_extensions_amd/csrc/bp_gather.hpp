@@ -52,19 +52,35 @@ constexpr int kGatherLanes = 64;    // channel intervals per workgroup (one lane
 constexpr int kGatherOut = kGatherLanes - 1;  // output channels per workgroup
 constexpr double kGatherEps = 1.0 / 32;
 
+// The first 32 bytes of an anchor (all the gather reads).  For a policy with
+// kGatherFrac the whole channels of its position are moved into is0 and fc
+// holds the fraction, so a pixel's position is rounded at the size of its
+// offset from the anchor (as the stream kernel's are) and not of the distance
+// to the tile's first channel.
+struct alignas(16) GatherAnchor {
+    uint4 lo, hi;
+};
+
 // anchors[view][tile] of 16 x 16 tiles: the FP64 per-(tile, view) geometry,
 // evaluated once per call.
 template <class Geo>
 __global__ void bp_anchor_table_kernel(const typename Geo::Problem P, const typename Geo::Tables T,
-                                       int tiles_x, int ntiles, typename Geo::Anchor* __restrict__ out)
+                                       int tiles_x, int ntiles, GatherAnchor* __restrict__ out)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int v = blockIdx.y;
     if (t >= ntiles) return;
     const TileFrame F(t, tiles_x, P.nx, P.ny, kGatherTile, kGatherTile);
-    out[static_cast<size_t>(v) * ntiles + t] =
+    typename Geo::Anchor A =
         Geo::anchor(P, T, F, v, F.x0 - F.ic, F.x0 + kGatherTile - 1 - F.ic, F.y0 - F.jc,
                     F.y0 + kGatherTile - 1 - F.jc);
+    if constexpr (Geo::kGatherFrac) {
+        A.is0 += A.whole;
+        A.fc = A.frac;
+    }
+    GatherAnchor G;
+    __builtin_memcpy(&G, &A, sizeof(G));
+    out[static_cast<size_t>(v) * ntiles + t] = G;
 }
 
 // dst[b][x][y] = src[b][y][x] (the image seen column by column).
@@ -89,7 +105,7 @@ template <class Geo>
 struct GatherLaunch {
     typename Geo::Problem P;
     typename Geo::Tables T;
-    const typename Geo::Anchor* anchors;  // [na][tiles_x * tiles_y]
+    const GatherAnchor* anchors;          // [na][tiles_x * tiles_y]
     const float* img;                     // [nbatch][ny][nx]
     const float* imgT;                    // [nbatch][nx][ny]
     float* proj;                          // [nbatch][na][ns]
@@ -160,7 +176,8 @@ void bp_gather_t_kernel(const GatherLaunch<Geo> L)
     using Anchor = typename Geo::Anchor;
     constexpr int V = kGatherViews, K = S::kTiles, NG = S::kGroups;
     static_assert(sizeof(Anchor) % 16 == 0 && sizeof(Anchor) >= 32 &&
-                      offsetof(Anchor, inside) < 32 && offsetof(Anchor, is0) < 32,
+                      offsetof(Anchor, inside) < 32 && offsetof(Anchor, is0) < 32 &&
+                      offsetof(Anchor, fc) < 32,
                   "the gather reads an anchor's first 32 bytes");
     static_assert(kGatherViews * S::kTiles <= 256, "one thread per staged anchor");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -357,10 +374,10 @@ void bp_gather_t_kernel(const GatherLaunch<Geo> L)
                 uint4 q0 = make_uint4(0u, 0u, 0u, 0u), q1 = q0;
                 if (v0 + v < P.na && tw < tw_max) {
                     const int tile = frame ? tw * L.tiles_x + tu : tu * L.tiles_x + tw;
-                    const uint4* a = reinterpret_cast<const uint4*>(
-                        L.anchors + static_cast<size_t>(v0 + v) * L.tiles_x * L.tiles_y + tile);
-                    q0 = a[0];
-                    q1 = a[1];
+                    const GatherAnchor& a =
+                        L.anchors[static_cast<size_t>(v0 + v) * L.tiles_x * L.tiles_y + tile];
+                    q0 = a.lo;
+                    q1 = a.hi;
                 }
                 uint4* d = reinterpret_cast<uint4*>(sanc) + 2 * tid;
                 d[0] = q0;
@@ -416,10 +433,20 @@ void bp_gather_t_kernel(const GatherLaunch<Geo> L)
                 const float fu = static_cast<float>(u0 + r - uc);
                 const float fw = static_cast<float>(
                     w - min((w & ~(kGatherTile - 1)) + kGatherTile / 2, wcl));
-                float f, wt;
+                float f, wt, frac = 0.0f;
+                int s = A.is0;
+                if constexpr (Geo::kGatherFrac) {
+                    frac = A.fc;
+                    A.fc = 0.0f;
+                }
                 Geo::pixel(Pg, A, frame ? fu : fw, frame ? fw : fu, f, wt);
+                if constexpr (Geo::kGatherFrac) {
+                    const float whole = floorf(f);
+                    s += static_cast<int>(whole);
+                    f = frac + (f - whole);  // in [0, 2)
+                }
                 const float fr = __builtin_amdgcn_fractf(f);
-                const int s = A.is0 + static_cast<int>(f);
+                s += static_cast<int>(f);
                 // the forward's edge rule, only for tiles that reach past the
                 // detector (few, and the same for most lanes of a wave)
                 if (!A.inside) wt = on_detector(s, fr, P.ns) ? wt : 0.0f;
@@ -460,12 +487,11 @@ void bp_gather_t_kernel(const GatherLaunch<Geo> L)
 // Host side: workspace bytes and the launch sequence (anchor table, the
 // transposed image, the gather).  ws: caller-provided workspace of
 // gather_workspace_bytes(...) bytes, or null to allocate it on the stream.
-template <class Anchor>
 inline size_t gather_workspace_bytes(int na, int nx, int ny, int nbatch)
 {
     const size_t ntiles = static_cast<size_t>((nx + kGatherTile - 1) / kGatherTile) *
                           ((ny + kGatherTile - 1) / kGatherTile);
-    const size_t anc = (na * ntiles * sizeof(Anchor) + 255) & ~static_cast<size_t>(255);
+    const size_t anc = (na * ntiles * sizeof(GatherAnchor) + 255) & ~static_cast<size_t>(255);
     return anc + static_cast<size_t>(nbatch) * nx * ny * sizeof(float);
 }
 
@@ -489,7 +515,6 @@ int launch_bp_gather_t(const typename Geo::Problem& P, const typename Geo::Table
                        const float* img, float* proj, int nbatch, double scale, void* ws,
                        hipStream_t st)
 {
-    using Anchor = typename Geo::Anchor;
     GatherLaunch<Geo> L{};
     L.P = P;
     L.T = T;
@@ -500,14 +525,14 @@ int launch_bp_gather_t(const typename Geo::Problem& P, const typename Geo::Table
     L.img = img;
     L.proj = proj;
     const int ntiles = L.tiles_x * L.tiles_y;
-    const size_t bytes = gather_workspace_bytes<Anchor>(P.na, P.nx, P.ny, nbatch);
+    const size_t bytes = gather_workspace_bytes(P.na, P.nx, P.ny, nbatch);
     void* own = nullptr;
     if (!ws) {
         CTR_HIP(ctr::ws_alloc(&own, bytes, st));
         ws = own;
     }
-    auto* table = static_cast<Anchor*>(ws);
-    const size_t anc = (static_cast<size_t>(P.na) * ntiles * sizeof(Anchor) + 255) &
+    auto* table = static_cast<GatherAnchor*>(ws);
+    const size_t anc = (static_cast<size_t>(P.na) * ntiles * sizeof(GatherAnchor) + 255) &
                        ~static_cast<size_t>(255);
     float* imgT = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) + anc);
     L.anchors = table;

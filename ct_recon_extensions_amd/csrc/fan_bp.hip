@@ -180,6 +180,13 @@ int fan_problem(const ctr_geom& g, int TW, int TH, FanProblem& P, int& lmax, boo
     P.nx = static_cast<int>(g.nx);
     P.ny = static_cast<int>(g.ny);
     const double k = g.dsd / g.ds;
+    P.kd = k;
+    P.idsd = 1.0 / g.dsd;
+    P.dxd2 = static_cast<float>(g.dx * g.dx / (g.dsd * g.dsd));
+    // 3.5 pixels at up to k dx / distance channels a pixel
+    P.roff = static_cast<float>(
+        std::ceil(3.6 * k * std::fabs(g.dx) / std::max(fan_min_distance(g, 16, 16), 1e-3 * g.dso)) +
+        1.0);
     P.k = static_cast<float>(k);
     P.p1 = static_cast<float>(-1.0 / (3 * k * k));
     P.p2 = static_cast<float>(1.0 / (5 * k * k * k * k));
@@ -200,6 +207,25 @@ int fan_problem(const ctr_geom& g, int TW, int TH, FanProblem& P, int& lmax, boo
     const double umax = std::tan(0.5 * ang);
     exact = (k * std::pow(umax, 7) / 7 > 2e-7) || (std::pow(umax, 6) > 5e-8) || umax > 0.25;
     return CTR_OK;
+}
+
+// What the run polynomials leave out (FanRun), with e = dx / distance, d <= 3.5
+// pixels, and the largest values of the angle terms: 22 d^4-units of 0.25 k e^4
+// channels and 10.5 d^3-units of 4 e^3 of the weight (short), 33 d^5-units of 0.25
+// k e^5 and 22 d^4-units of 5 e^4 (long).  Admitted: 1e-6 channel (a position in a
+// 64-channel span rounds to 4e-6) and 4e-7 of the weight, at the pixels nearest
+// the source; at the rotation centre of a scan whose image fills the field of
+// view they are 9 (e^4) and 5 (e^3) times smaller.  A 512^2 image over 358 mm at
+// 595 mm takes the short form, 192^2 the long one; coarser pixels stay on the
+// engine kernel.
+int fan_run_order(const ctr_geom& g)
+{
+    const double lmin = fan_min_distance(g, kStreamTile, kStreamTile);
+    if (!(lmin > 0)) return 0;
+    const double e = std::fabs(g.dx) / lmin, k = g.dsd / g.ds, e3 = e * e * e;
+    if (5.5 * k * e3 * e <= 1e-6 && 42.0 * e3 <= 4e-7) return 1;
+    if (8.3 * k * e3 * e * e <= 1e-6 && 110.0 * e3 * e <= 4e-7) return 2;
+    return 0;
 }
 
 namespace {
@@ -300,6 +326,19 @@ int fan_bp_f32(const ctr_geom& g, const float* proj, float* img, int nbatch, con
         if (rc) return rc;
     }
     const FanTables T{xpos, ypos, sc};
+    const int order = cfg.tile == 0 && cfg.vchunk == 0 && cfg.nb == 0 && !exact &&
+                              stream_applies(lmax, g.na, g.ns)
+                          ? fan_run_order(g)
+                          : 0;
+    if (order) {
+        const auto launch = [&](auto L) {
+            L.P = P;
+            L.scale = scale;
+            L.img = img;
+            return launch_stream_batch(L, T, proj, nbatch, lmax, st);
+        };
+        return order == 1 ? launch(StreamLaunch<FanRun<false>>{}) : launch(StreamLaunch<FanRun<true>>{});
+    }
     const int nb = engine_nb(cfg.nb ? cfg.nb : auto_nb(nbatch), g.na, g.ns);
 #define CTR_FAN_NB(TW_, TH_)                                                                   \
     switch (nb) {                                                                              \
@@ -321,7 +360,7 @@ int fan_bp_f32(const ctr_geom& g, const float* proj, float* img, int nbatch, con
 }
 
 // float32 transpose: the gather form (bp_gather.hpp), deterministic in both
-// modes.  ws: caller workspace of gather_workspace_bytes<FanAnchor>(...)
+// modes.  ws: caller workspace of gather_workspace_bytes(...)
 // bytes, or null for a stream-ordered allocation.
 int fan_bpt_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, const double* xpos,
                 const double* ypos, const double* sc, double scale, bool det, void* ws,

@@ -669,7 +669,22 @@ int fpt_typed(const ctr_geom& g, const T* proj, T* img, int nbatch, const double
         if (fpt_engine_applies(g) && g.nx >= 3 && g.ny >= 3) {
             // interior on the engine, then the border pixels exactly
             const int s = static_cast<int>(stride);
-            int rc;
+            int rc = CTR_OK;
+            FpProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
+                        static_cast<int>(g.ny), nbatch, g.dx, g.dy};
+            if (stream_applies(48, g.na, g.ns)) {
+                StreamLaunch<FptGeo> S{};
+                S.P = FptProblem{P.ns, P.na, P.nx, P.ny};
+                S.scale = 1.0;
+                S.img = img;
+                const FptTables tab{w, pos, usex, s};
+                // a caller's workspace means that nothing may be allocated
+                rc = ws ? launch_stream_batch<FptGeo, true>(S, tab, proj, nbatch, 48, st)
+                        : launch_stream_batch<FptGeo>(S, tab, proj, nbatch, 48, st);
+                if (rc) return rc;
+                return nbatch >= 8 ? launch_fpt_border<8>(P, proj, img, w, pos, usex, s, ws, st)
+                                   : launch_fpt_border<1>(P, proj, img, w, pos, usex, s, ws, st);
+            }
             const int nb = engine_nb(nbatch >= 8 ? 8 : nbatch >= 4 ? 4 : nbatch, g.na, g.ns);
             // the applicability bound keeps a tile-view's span within
             // 30 max(dx,dy)/ds + 5 <= 35 channels: 48-channel rows when the
@@ -679,8 +694,6 @@ int fpt_typed(const ctr_geom& g, const T* proj, T* img, int nbatch, const double
             else if (nb >= 2) rc = launch_fpt_engine<2, 64>(g, proj, img, nbatch, w, pos, usex, s, st);
             else rc = launch_fpt_engine<1, 64>(g, proj, img, nbatch, w, pos, usex, s, st);
             if (rc) return rc;
-            FpProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
-                        static_cast<int>(g.ny), nbatch, g.dx, g.dy};
             return nbatch >= 8 ? launch_fpt_border<8>(P, proj, img, w, pos, usex, s, ws, st)
                                : launch_fpt_border<1>(P, proj, img, w, pos, usex, s, ws, st);
         }

@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstddef>
 
+#include "bp_stream.hpp"
 #include "tile_common.hpp"
 
 namespace ctr {
@@ -24,9 +25,17 @@ struct alignas(16) FptAnchor {
     float inv_o1;  // 1/|o1|
     float wv;      // the view's weight |dy/cos| or |dx/sin|
     int is0;
-    int inside;    // unused by the custom taps (kept for the engine)
+    int inside;    // whole tile strictly inside the detector
     int nch;       // channels from is0 the tile's taps can touch (one of margin)
-    int pad[3];
+    float frac;    // mid at the anchor pixel is is0 + whole + frac
+    int whole;
+    int pad;
+};
+
+// The part of an anchor the stream kernel's pixels read, in one LDS line.
+struct alignas(16) FptStreamAnchor {
+    float a, b, frac, inv_o1, rest, wv;  // rest = 1 - 1/|o1|
+    int is0, nch;                        // nch: FptAnchor::nch | whole << 16
 };
 
 struct FptProblem {
@@ -75,9 +84,12 @@ struct FptGeo {
         A.inv_o1 = static_cast<float>(1.0 / fabs(o1));
         A.wv = static_cast<float>(T.weights[view]);
         A.is0 = is0;
-        A.inside = 1;
+        // every tap of the tile on the detector
+        A.inside = midc + lo >= 0.25 && midc + hi <= P.ns - 1.25 ? 1 : 0;
         A.nch = static_cast<int>(floor(midc + hi)) + 3 - is0;
-        A.pad[0] = A.pad[1] = A.pad[2] = 0;
+        A.whole = static_cast<int>(floor(midc)) - is0;
+        A.frac = static_cast<float>(midc - floor(midc));
+        A.pad = 0;
         return A;
     }
 
@@ -91,6 +103,32 @@ struct FptGeo {
         const float io = A.inv_o1;
         w0 = fmaxf(0.0f, fmaf(-fr, io, 1.0f)) * A.wv;        // channel floor(mid)
         w1 = fmaxf(0.0f, fmaf(fr - 1.0f, io, 1.0f)) * A.wv;  // channel floor(mid) + 1
+    }
+
+    // runs of the stream kernel (bp_stream.hpp): mid is exactly linear
+    using StreamAnchor = FptStreamAnchor;
+    static constexpr int kRunDegree = 1;
+    __device__ __forceinline__ static StreamAnchor pack(const Anchor& A)
+    {
+        return StreamAnchor{A.a, A.b, A.frac, A.inv_o1, 1.0f - A.inv_o1, A.wv, A.is0,
+                            A.nch | A.whole << 16};
+    }
+    __device__ __forceinline__ static RunPoly run(const Problem&, const StreamAnchor& A, float fi,
+                                                  float fj)
+    {
+        RunPoly R{};
+        // |a| <= 1 (fpt_engine_applies): a run stays within 3.5 channels
+        run_base(R, A.nch >> 16, A.frac, fmaf(A.a, fi, A.b * fj), 5.0f);
+        R.c1 = A.a;
+        R.w0 = A.wv;
+        return R;
+    }
+    // wv: the view's weight (0 for a half without a view)
+    __device__ __forceinline__ static void stream_weights(const StreamAnchor& A, float fr, float wv,
+                                                          float& w0, float& w1)
+    {
+        w0 = fmaxf(0.0f, fmaf(-fr, A.inv_o1, 1.0f)) * wv;
+        w1 = fmaxf(0.0f, fmaf(fr, A.inv_o1, A.rest)) * wv;
     }
 };
 

@@ -9,6 +9,7 @@
 // differences.  Output scale is the signed orbit (src/bp_par_2d.cc:83).
 #include "bp_engine.hpp"
 #include "bp_gather.hpp"
+#include "bp_stream.hpp"
 #include "ctr_common.hpp"
 #include "tile_common.hpp"
 
@@ -24,6 +25,14 @@ struct alignas(16) ParAnchor {
     int is0;     // first staged channel
     int inside;  // whole tile strictly inside the detector
     int nch;     // channels from is0 the tile's taps can touch (one of margin)
+    float frac;  // the anchor's channel position is is0 + whole + frac
+    int whole;
+};
+
+// The part of an anchor the stream kernel's pixels read, in one LDS line.
+struct alignas(16) ParStreamAnchor {
+    float a, b, frac, off;  // off: channels a run stays within of its centre
+    int is0, nch;           // nch: ParAnchor::nch | whole << 16
     int pad[2];
 };
 
@@ -53,7 +62,8 @@ __device__ inline ParAnchor par_anchor(const ParProblem& P, const double* __rest
     A.is0 = is0;
     A.inside = (sc + lo >= 0.25 && sc + hi <= P.ns - 1.25) ? 1 : 0;
     A.nch = static_cast<int>(floor(sc + hi)) + 3 - is0;
-    A.pad[0] = A.pad[1] = 0;
+    A.whole = static_cast<int>(floor(sc)) - is0;
+    A.frac = static_cast<float>(sc - floor(sc));
     return A;
 }
 
@@ -67,6 +77,7 @@ struct ParGeo {
     using Problem = ParProblem;
     using Tables = ParTables;
     using Anchor = ParAnchor;
+    static constexpr bool kGatherFrac = true;
     __device__ static Anchor anchor(const Problem& P, const Tables& T, const TileFrame& F,
                                     int view, int ilo, int ihi, int jlo, int jhi)
     {
@@ -77,6 +88,23 @@ struct ParGeo {
     {
         f = fmaf(A.a, fi, fmaf(A.b, fj, A.fc));
         w = 1.0f;
+    }
+    // runs of the stream kernel (bp_stream.hpp): exactly linear
+    using StreamAnchor = ParStreamAnchor;
+    static constexpr int kRunDegree = 1;
+    __device__ __forceinline__ static StreamAnchor pack(const Anchor& A)
+    {
+        return StreamAnchor{A.a,   A.b,   A.frac, ceilf(4.0f * fabsf(A.a)) + 1.0f,
+                            A.is0, A.nch | A.whole << 16, {0, 0}};
+    }
+    __device__ __forceinline__ static RunPoly run(const Problem&, const StreamAnchor& A, float fi,
+                                                  float fj)
+    {
+        RunPoly R{};
+        run_base(R, A.nch >> 16, A.frac, fmaf(A.a, fi, A.b * fj), A.off);
+        R.c1 = A.a;
+        R.w0 = 1.0f;
+        return R;
     }
     // Level line s = s_star in pixel-index coordinates: the tables are linear
     // in the index (xcos[ix][view] = x0 cos + ix dx cos), so
@@ -257,6 +285,13 @@ int par_bp(const ctr_geom& g, int dtype, const void* proj, void* img, int nbatch
     const ParTables T{xcos, ysin};
     L.proj = static_cast<const float*>(proj);
     L.img = static_cast<float*>(img);
+    if (stream_applies(L.lmax, g.na, g.ns)) {
+        StreamLaunch<ParGeo> S{};
+        S.P = L.P;
+        S.scale = g.orbit;
+        S.img = L.img;
+        return launch_stream_batch(S, T, L.proj, nbatch, L.lmax, st);
+    }
     const int nb = engine_nb(
         nbatch >= 16 ? 16 : nbatch >= 8 ? 8 : nbatch >= 4 ? 4 : nbatch >= 2 ? 2 : 1, g.na, g.ns);
     switch (nb) {

@@ -39,13 +39,19 @@ struct RaggedDesc {
     double scale;
     int tiles_x, tiles_y;
     int lmax, vchunk;
-    int variant;  // 4 * exact + span class (0: 64, 1: 128, 2: 256 channels)
-    int pad;
+    // 4 * exact + span class (0: 64, 1: 128, 2: 256 channels) of the engine
+    // tile, or 7 + fan_run_order (8 short, 9 long runs) of the stream tile
+    int variant;
+    int wave_bytes;  // stream tile: LDS per wave
 };
 
 struct RaggedItem {
     int prob, tile;
 };
+
+// Anchors a wave of the stream tile keeps at once: 4 of the 10 KB of LDS it has
+// at sixteen waves a CU (more views are taken in rounds).
+constexpr int kRaggedViews = 128;
 
 __global__ void ragged_clear_kernel(unsigned int* counter) { counter[0] = 0u; }
 
@@ -71,6 +77,16 @@ __device__ __forceinline__ void ragged_run_item(const RaggedDesc& D, int tile, u
 #undef CTR_RAGGED_CASE
 }
 
+template <bool LONG>
+__device__ __forceinline__ void ragged_run_stream(const RaggedDesc& D, int tile, int nwaves,
+                                                  unsigned char* smem)
+{
+    StreamLaunch<FanRun<LONG>> L{D.P,      1,      D.tiles_x,      D.tiles_y,
+                                 D.lmax,   D.vchunk, kRaggedViews, D.wave_bytes,
+                                 D.scale,  D.proj,   D.img};
+    stream_tile<FanRun<LONG>, 1, 8, true>(D.T, L, tile, 0, nwaves, smem);
+}
+
 // Persistent kernel: every workgroup loops until the item counter passes
 // nitems (each workgroup exits after at most one failed fetch, so the grid
 // always drains).  stamps (optional): per-workgroup first and last
@@ -91,7 +107,16 @@ __attribute__((amdgpu_waves_per_eu(4, 4))) void ragged_fan_bp_kernel(
         if (it >= nitems) break;
         const RaggedItem item = items[it];
         const int prob = uniform_i(item.prob), tile = uniform_i(item.tile);
-        ragged_run_item<TW, TH>(descs[prob], tile, smem);
+        const RaggedDesc& D = descs[prob];
+        if constexpr (TW == kStreamTile && TH == kStreamTile) {
+            const int variant = uniform_i(D.variant);
+            if (variant >= 8) {
+                if (variant == 8) ragged_run_stream<false>(D, tile, blockDim.x >> 6, smem);
+                else ragged_run_stream<true>(D, tile, blockDim.x >> 6, smem);
+                continue;
+            }
+        }
+        ragged_run_item<TW, TH>(D, tile, smem);
     }
     if (stamps && threadIdx.x == 0) {
         stamps[2 * blockIdx.x] = t0;
@@ -238,9 +263,23 @@ int ctr_ragged_fan_bp_plan(const ctr_ragged_problem* probs, int nprob, int tile,
             D.lmax = lmax;
             D.vchunk = vc;
             D.variant = (exact ? 4 : 0) + cls;
+            D.wave_bytes = 0;
+            const int order =
+                tile == 0 && !exact && lmax <= kStreamMaxPitch ? fan_run_order(q.g) : 0;
+            if (order) {
+                D.variant = 7 + order;
+                D.lmax = (lmax + 15) / 16 * 16;  // the staged spans' pitch
+                const int wave_lds = static_cast<int>(lds_budget) / (block / 64);
+                const int fit = (wave_lds - kRaggedViews * 32) / (2 * D.lmax * 4);
+                D.vchunk = std::max(2, std::min(vchunk, fit) / 2 * 2);
+                D.wave_bytes = stream_wave_bytes(1, 1, D.lmax, D.vchunk, kRaggedViews);
+                vc = 1;
+                lds = std::max(lds, static_cast<size_t>(block / 64) * D.wave_bytes);
+            }
             lds = std::max(lds, anchor_bytes + 2 * static_cast<size_t>(vc) * lrow * sizeof(float));
-            // exact tiles evaluate atanf per pixel-view: roughly 1.6x the work
-            item_cost[i] = static_cast<double>(q.g.na) * TW * TH * (exact ? 1.6 : 1.0);
+            // exact tiles evaluate atanf per pixel-view: roughly 1.6x the work;
+            // runs roughly 0.65x
+            item_cost[i] = static_cast<double>(q.g.na) * TW * TH * (exact ? 1.6 : order ? 0.65 : 1.0);
             pv += static_cast<double>(q.g.na) * q.g.nx * q.g.ny;
             nitems += static_cast<long long>(D.tiles_x) * D.tiles_y;
         }

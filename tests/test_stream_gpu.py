@@ -1,0 +1,166 @@
+"""The run-polynomial BP kernels (bp_stream.hpp) at the sizes where they can go
+wrong, against the oracle: every group size and its remainders (16, 8, 4, 2, 1
+slices), fewer views than waves and view counts that split unevenly, images
+smaller than a tile and with partial tiles, tiles that reach past the detector,
+both run orders and the geometries that stay on the engine kernel, spans of one
+and of two DMA rows.  Tolerance: the suite's 1e-5 relative L2 (positions are
+within a few 1e-6 channel, i.e. a few 1e-6 on N(0, 1) sinograms)."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.conftest import randn, rel_l2
+
+pytestmark = pytest.mark.gpu
+TOL32 = 1e-5
+
+
+@pytest.fixture(scope="module")
+def F():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import ct_recon_extensions_amd as F
+    from ct_recon_extensions_amd import _lib
+    _lib.load()
+    return F
+
+
+def kwargs(g, fan):
+    kw = dict(img_shape=[g["ny"], g["nx"]], img_space=[g["dy"], g["dx"]],
+              proj_shape=[g["na"], g["ns"]], channel_space=g["ds"],
+              img_offset=[g["offset_y"], g["offset_x"]], channel_offset=g["offset_s"],
+              orbit_start=g["orbit_start"], orbit=g["orbit"])
+    return dict(kw, dso=g["dso"], dsd=g["dsd"]) if fan else kw
+
+
+def geom(n, na, ns, dx, ds, fan=True, offset_s=0.25, ny=None):
+    g = dict(nx=n, ny=ny or n, na=na, ns=ns, dx=dx, dy=dx, ds=ds, offset_x=0.3, offset_y=-0.7,
+             offset_s=offset_s, orbit_start=0.1, orbit=(2 if fan else 1) * math.pi / na)
+    return dict(g, dso=595.0, dsd=1085.6) if fan else g
+
+
+# (geometry, slices)
+FAN = [
+    (geom(64, 90, 96, 0.7, 1.3), 1), (geom(64, 90, 96, 0.7, 1.3), 2),
+    (geom(64, 90, 96, 0.7, 1.3), 3), (geom(50, 45, 80, 0.7, 1.3, ny=37), 5),
+    (geom(50, 45, 80, 0.7, 1.3, ny=37), 9), (geom(33, 61, 70, 0.7, 1.3), 10),
+    (geom(33, 61, 70, 0.7, 1.3), 18),
+    (geom(40, 5, 64, 0.7, 1.3), 1), (geom(40, 7, 64, 0.7, 1.3), 8),    # fewer views than waves
+    (geom(7, 33, 40, 0.7, 1.3), 4), (geom(17, 130, 40, 0.7, 1.3), 16),  # partial tiles
+    (geom(96, 60, 40, 0.7, 1.3), 1), (geom(96, 60, 40, 0.7, 1.3), 4),   # truncated detector
+    (geom(96, 60, 41, 0.7, 1.3, offset_s=11.0), 8),
+    (geom(96, 60, 40, 0.7, 1.3), 2), (geom(96, 60, 40, 0.7, 1.3), 16),
+    (geom(48, 70, 120, 1.6, 1.3), 1), (geom(48, 70, 120, 1.6, 1.3), 6),  # long runs
+    (geom(32, 50, 64, 5.0, 2.0), 2),                                     # engine kernel
+    (geom(64, 40, 400, 0.7, 0.35), 1), (geom(64, 40, 400, 0.7, 0.35), 4),  # two DMA rows a span
+    (geom(64, 40, 400, 0.7, 0.35), 16),
+    (geom(20, 1537, 48, 0.7, 1.3), 2),  # more views than the waves hold
+    (geom(20, 1100, 48, 0.7, 1.3), 16), (geom(20, 1536, 48, 0.7, 1.3), 8),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FAN)))
+def test_fan_bp_stream_matches_oracle(F, case):
+    g, n = FAN[case]
+    og = O.geom(**g)
+    t = O.fan_prep(og)
+    proj = randn(900 + case, (n, g["na"], g["ns"]))
+    out = F.fan_backprojection_2d(torch.from_numpy(proj).cuda(), **kwargs(g, True)).cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.fan_bp(og, proj[b], t)) < TOL32, b
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 7, 16, 17])
+@pytest.mark.parametrize("ns,offset_s", [(60, 0.0), (23, 5.5)])
+def test_par_bp_stream_matches_oracle(F, n, ns, offset_s):
+    g = geom(45, 50, ns, 1.0, 1.0, fan=False, offset_s=offset_s, ny=38)
+    og = O.geom(**g)
+    t = O.par_prep(og)
+    proj = randn(950 + n, (n, g["na"], ns))
+    out = F.parallel_backprojection_2d(torch.from_numpy(proj).cuda(),
+                                       **kwargs(g, False)).cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.par_bp(og, proj[b], t)) < TOL32, b
+
+
+@pytest.mark.parametrize("n", [1, 2, 4])
+@pytest.mark.parametrize("ns", [24, 25, 26, 27])
+def test_last_channels_of_the_last_view(F, n, ns):
+    """One tile, one view a wave, the last view's taps ending at channel ns - 1:
+    a 16-byte load there reaches past the sinogram's end, and the channels
+    before the end still count."""
+    g = geom(16, 8, ns, 1.0, 1.0, fan=False)
+    last = g["orbit_start"] + 7 * g["orbit"]
+    reach = ((7.5 + abs(g["offset_x"])) * abs(math.cos(last))
+             + (7.5 + abs(g["offset_y"])) * abs(math.sin(last)))
+    g["offset_s"] = ns - 1.3 - reach - (ns - 1) / 2
+    og = O.geom(**g)
+    t = O.par_prep(og)
+    proj = randn(980 + ns, (n, 8, ns))
+    out = F.parallel_backprojection_2d(torch.from_numpy(proj).cuda(),
+                                       **kwargs(g, False)).cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.par_bp(og, proj[b], t)) < TOL32, b
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 8, 11, 17])
+@pytest.mark.parametrize("ns", [80, 31])
+def test_fpt_stream_matches_oracle_and_noalloc(F, n, ns):
+    from ct_recon_extensions_amd import _lib
+    from ct_recon_extensions_amd.geometry import ParallelProjection2DParam, device_tables
+    g = geom(40, 50, ns, 1.0, 1.1, fan=False)
+    og = O.geom(**g)
+    t = O.fp_grad_prep(og)
+    proj = randn(970 + n, (n, g["na"], ns))
+    x = torch.from_numpy(proj).cuda()
+    out = F.parallel_projection_2d_grad(x, **kwargs(g, False))
+    for b in range(n):
+        assert rel_l2(out[b].cpu().numpy(), O.fp_grad(og, proj[b], t)) < TOL32, b
+    # the allocation-free entry point stages the same spans: the same bits
+    p = ParallelProjection2DParam(ns, g["na"], g["ds"], g["orbit"], g["offset_s"],
+                                  g["orbit_start"], 40, 40, 1.0, 1.0, g["offset_x"], g["offset_y"])
+    w, pos, usex = device_tables("fp_grad", p, x.device)
+    got = torch.empty_like(out)
+    _lib.call("ctr_fp_t_noalloc", C.byref(p.ctr()), 0, C.c_void_p(x.data_ptr()),
+              C.c_void_p(got.data_ptr()), n, C.c_void_p(w.data_ptr()), C.c_void_p(pos.data_ptr()),
+              C.c_void_p(usex.data_ptr()), 40,
+              C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(got, out)
+
+
+def test_nonfinite_samples_stay_in_their_pixels(F):
+    """inf and nan samples reach the pixels whose taps they are, as in the
+    engine kernel (an explicit launch shape), and no others."""
+    from ct_recon_extensions_amd import _lib
+    from ct_recon_extensions_amd.geometry import FanBackprojection2DParam, device_tables
+    g = geom(60, 37, 44, 0.7, 1.3)  # truncated: edge and inner tiles
+    proj = randn(990, (4, g["na"], g["ns"]))
+    proj[0, 3, 20], proj[1, 36, 43], proj[2, 0, 0] = np.inf, np.nan, -np.inf
+    x = torch.from_numpy(proj).cuda()
+    out = F.fan_backprojection_2d(x, **kwargs(g, True))
+    p = FanBackprojection2DParam(g["ns"], g["na"], g["ds"], g["orbit"], g["offset_s"],
+                                 g["orbit_start"], 60, 60, 0.7, 0.7, 0.3, -0.7, 595.0, 1085.6)
+    tabs = device_tables("fan", p, x.device)
+    ref = torch.empty_like(out)
+    _lib.call("ctr_fan_bp_ex", C.byref(p.ctr()), 0, C.c_void_p(x.data_ptr()),
+              C.c_void_p(ref.data_ptr()), 4, *(C.c_void_p(t.data_ptr()) for t in tabs), p.scale,
+              C.byref(_lib.CtrFanBpLaunch(0, 6, 4)),
+              C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(torch.isfinite(out), torch.isfinite(ref))
+    assert not torch.isfinite(out[:3]).all() and torch.isfinite(out[3]).all()
+    one = F.fan_backprojection_2d(x[1:2], **kwargs(g, True))
+    assert torch.equal(torch.isfinite(one), torch.isfinite(ref[1:2]))
+
+
+def test_workspace_is_given_back(F):
+    from ct_recon_extensions_amd import _lib
+    g = geom(64, 90, 96, 0.7, 1.3)
+    x = torch.from_numpy(randn(999, (4, 90, 96))).cuda()
+    a = F.fan_backprojection_2d(x, **kwargs(g, True))
+    torch.cuda.synchronize()
+    _lib.call("ctr_release_workspace")
+    assert torch.equal(a, F.fan_backprojection_2d(x, **kwargs(g, True)))
