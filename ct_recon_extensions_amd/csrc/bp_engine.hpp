@@ -40,6 +40,12 @@ __device__ __forceinline__ float uniform_f(float x)
 }
 __device__ __forceinline__ int uniform_i(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+// x of lane `lane` (uniform) of the wave, through a scalar register.
+__device__ __forceinline__ float lane_value(float x, int lane)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
 // Views per LDS round for the forward kernel: the most (up to one anchor
 // chunk) whose two span buffers and the anchors fit a quarter of a CU's
 // 160 KB, i.e. four workgroups per CU (fewer views per round means a barrier

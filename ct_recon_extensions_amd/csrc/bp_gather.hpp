@@ -113,12 +113,6 @@ struct GatherLaunch {
     double scale;
 };
 
-// x of lane `lane` (uniform) of the wave, through a scalar register.
-__device__ __forceinline__ float lane_value(float x, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
-
 // One linear constraint of a lane's candidates along a row: w >= A + B u
 // (lower) or w <= A + B u (upper); none = no constraint from this line.
 struct GatherBound {

@@ -1,7 +1,9 @@
 // Ray-driven parallel-beam forward projection for gfx950 and its
 // gather-form transpose.
 //
-// FP (fp_kernel): one thread per ray (view, channel) for NB slices; a
+// FP (fp_stream.hpp; float32): waves stream image rows through their own LDS,
+// one ray a lane for several views and slices.  fp_kernel (float64, and spans
+// beyond that kernel's): one thread per ray (view, channel) for NB slices; a
 // workgroup covers 256 consecutive channels of one view, so the sinogram row
 // is written coalesced.  The ray marches the rows of the image (x-branch) or
 // its columns (y-branch); the branch, the start position and the step of
@@ -26,6 +28,7 @@
 // along the marched axis keep one side only (src/fp_par_2d.cc:360-368).
 #include "bp_engine.hpp"
 #include "ctr_common.hpp"
+#include "fp_stream.hpp"
 #include "fpt_geom.hpp"
 #include "tile_common.hpp"
 
@@ -37,11 +40,6 @@
 #include <unordered_map>
 
 namespace ctr {
-
-struct FpProblem {
-    int ns, na, nx, ny, nbatch;
-    double dx, dy;
-};
 
 // Transposed copy src[b][iy][ix] -> dst[b][ix][iy] through a 32x33 LDS tile.
 template <typename T>
@@ -120,186 +118,6 @@ __global__ __launch_bounds__(256) void fp_kernel(const T* __restrict__ img,
         if (b < nb)
             proj[(static_cast<size_t>(b0 + b) * P.na + a) * P.ns + s] =
                 static_cast<T>(static_cast<double>(sum[b]) * dw);
-}
-
-// FP with LDS-staged image rows (float32).  A workgroup owns up to 256
-// consecutive channels (one per thread) of V consecutive views and NB
-// slices, and marches the rows of the image (x-branch views) or of its
-// transpose (y-branch views) in chunks of kFpRows: per chunk it stages, for
-// all NB slices, the span of columns its rays can touch (DMA from global
-// straight into LDS, zero outside the row; slice rows kFpSpan words apart),
-// then every thread advances its V rays through those rows.  Two chunk
-// buffers alternate: the DMAs of chunk h + 1 are issued before the rays walk
-// chunk h, so their latency hides behind that walk and one barrier per chunk
-// separates the two.  A staged pixel is read by ~V rays instead of every view
-// re-reading the image through L1/L2, and a ray's two taps for a pair of
-// slices come from one ds_read2st64_b32.  Each ray keeps the reference's FP64
-// position accumulation (x += offset per row) and inclusion test; the lerp
-// and the sum are FP32.  Views of the other branch in the group take a second
-// pass.
-template <int NB, int V, int kFpRows, int kFpSpan>
-__global__ __launch_bounds__(256) void fp_lds_kernel(const float* __restrict__ img,
-                                                     const float* __restrict__ imgT,
-                                                     float* __restrict__ proj,
-                                                     const double* __restrict__ sincos,
-                                                     const double* __restrict__ bo,
-                                                     const int* __restrict__ usex, FpProblem P,
-                                                     int cpb)
-{
-    static_assert(NB % 2 == 0 || NB == 1, "slices are read in pairs");
-    constexpr int kChunk = kFpRows * NB * kFpSpan;  // floats of one chunk buffer
-    __shared__ __align__(16) float rows[2 * kChunk];
-    // the wave index is uniform: keeps the DMA's buffer descriptor in SGPRs
-    // (no per-lane waterfall around buffer_load ... lds)
-    const int tid = threadIdx.x, lane = tid & 63, wave = uniform_i(tid >> 6);
-    const int s0 = blockIdx.x * cpb, s = s0 + tid;
-    const int slast = min(s0 + cpb, P.ns) - 1;
-    const bool has_ray = tid < cpb && s < P.ns;
-    const int a0 = blockIdx.y * V;
-    const int b0 = blockIdx.z * NB;
-    const int nb = min(NB, P.nbatch - b0);
-    const size_t slice = static_cast<size_t>(P.nx) * P.ny;
-    // right tap through an offset the compiler cannot fold, so the slice
-    // pairs load as ds_read2st64_b32 (rows kFpSpan apart); at x == hi its
-    // weight u is 0 and it reads a staged zero
-    int one = 1;
-    asm volatile("" : "+v"(one));
-
-    for (int pass = 0; pass < 2; ++pass) {
-        const bool xb = pass == 0;
-        bool act[V];
-        int nact = 0;
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            const int a = a0 + v;
-            act[v] = a < P.na && (usex[a] != 0) == xb;
-            nact += act[v] ? 1 : 0;
-        }
-        if (nact == 0) continue;  // uniform
-        const int nsteps = xb ? P.ny : P.nx;
-        const int rowlen = xb ? P.nx : P.ny;
-        const float* src = xb ? img : imgT;
-        const double hi = rowlen - 1;
-        double x[V], off[V];
-        // view v's rays cover columns [clo[v] + k0 * coff[v], chi[v] + k0 * coff[v]]
-        // over rows k0 .. k0 + kFpRows - 1 (FP32 bounds: their error is far
-        // below the column of margin each side)
-        float clo[V], chi[V], coff[V];
-        float sum[V][NB];
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            const int a = min(a0 + v, P.na - 1);
-            const double* r = bo + 2 * static_cast<size_t>(a) * P.ns;
-            x[v] = has_ray ? r[2 * s] : 0.0;
-            off[v] = r[1];
-            const double blo = r[2 * s0], bhi = r[2 * slast];
-            const double drift = (kFpRows - 1) * off[v];
-            clo[v] = act[v] ? static_cast<float>(fmin(blo, bhi) + fmin(0.0, drift)) : 1e30f;
-            chi[v] = act[v] ? static_cast<float>(fmax(blo, bhi) + fmax(0.0, drift)) : -1e30f;
-            coff[v] = static_cast<float>(off[v]);
-#pragma unroll
-            for (int b = 0; b < NB; ++b) sum[v][b] = 0.0f;
-        }
-        // columns cmin .. cmin + 64 * nload - 1 of the chunk at row k0, or
-        // false when no ray of the chunk is on the image
-        auto span = [&](int k0, int& cmin, int& nload) -> bool {
-            const float k = static_cast<float>(k0);
-            float xmin = 1e30f, xmax = -1e30f;
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                xmin = fminf(xmin, fmaf(k, coff[v], clo[v]));
-                xmax = fmaxf(xmax, fmaf(k, coff[v], chi[v]));
-            }
-            if (xmax < -1.0f || xmin > static_cast<float>(hi) + 1.0f) return false;
-            // one column of margin each side; the right tap of a sample at
-            // x == nx-1 reads cmax + 1 (zero past the row); the host keeps
-            // cmax - cmin + 2 <= kFpSpan
-            cmin = max(0, static_cast<int>(floorf(xmin)) - 1);
-            const int cmax = min(rowlen - 1, static_cast<int>(floorf(xmax)) + 2);
-            nload = min((cmax - cmin + 65) / 64, kFpSpan / 64);
-            return true;
-        };
-        // rows (k0 + kk, slice b) -> buf[(kk * NB + b) * kFpSpan + c - cmin]
-        auto stage = [&](int k0, int cmin, int nload, float* buf) {
-            const int nr = min(kFpRows, nsteps - k0);
-            for (int e = wave; e < nr * NB; e += 4) {
-                const int kk = e / NB, b = e - kk * NB;
-                const float* rowp = src + static_cast<size_t>(b0 + b) * slice +
-                                    static_cast<size_t>(k0 + kk) * rowlen;
-                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                    const_cast<float*>(rowp), 0,
-                    b < nb ? static_cast<unsigned int>(rowlen) * 4u : 0u, 0x00020000);
-                float* dst = buf + e * kFpSpan;
-                for (int c = 0; c < nload; ++c)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                        rs, (__attribute__((address_space(3))) void*)(dst + 64 * c), 4,
-                        (cmin + 64 * c + lane) * 4, 0, 0, 0);
-            }
-        };
-        const int nchunks = (nsteps + kFpRows - 1) / kFpRows;
-        int cm = 0, nl = 0;
-        __syncthreads();  // the previous pass has finished reading both buffers
-        bool on = span(0, cm, nl);
-        if (on) stage(0, cm, nl, rows);
-        for (int h = 0; h < nchunks; ++h) {
-            const int k0 = h * kFpRows;
-            const int nr = min(kFpRows, nsteps - k0);
-            const float* cur = rows + (h & 1) * kChunk;
-            // this wave's DMAs of chunk h have landed (none of chunk h + 1 is
-            // issued yet); after the barrier every wave's have, and every
-            // wave is done with chunk h - 1, whose buffer takes chunk h + 1
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            int cm_next = 0, nl_next = 0;
-            bool on_next = false;
-            if (h + 1 < nchunks) {
-                on_next = span(k0 + kFpRows, cm_next, nl_next);
-                if (on_next) stage(k0 + kFpRows, cm_next, nl_next, rows + ((h + 1) & 1) * kChunk);
-            }
-            if (on && has_ray) {
-#pragma unroll 1
-                for (int kk = 0; kk < nr; ++kk) {
-                    const float* rk = cur + kk * NB * kFpSpan - cm;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        if (act[v] && x[v] >= 0 && x[v] <= hi) {
-                            // x >= 0: truncation is the floor, and the fraction is exact
-                            const int i1 = static_cast<int>(x[v]);
-                            const float u = static_cast<float>(__builtin_amdgcn_fract(x[v]));
-                            const float w0 = 1.0f - u;
-                            const float* q0 = rk + i1;
-                            const float* q1 = q0 + one;
-#pragma unroll
-                            for (int b = 0; b < NB; ++b)
-                                sum[v][b] = fmaf(u, q1[b * kFpSpan], fmaf(w0, q0[b * kFpSpan], sum[v][b]));
-                        }
-                        x[v] += off[v];
-                    }
-                }
-            } else {
-                // no ray of the chunk is on the image (or no ray here): only
-                // advance them
-#pragma unroll
-                for (int v = 0; v < V; ++v)
-                    for (int k = 0; k < nr; ++k) x[v] += off[v];
-            }
-            on = on_next;
-            cm = cm_next;
-        }
-        if (has_ray) {
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                if (!act[v]) continue;
-                const int a = a0 + v;
-                const double dw = xb ? fabs(P.dy / sincos[2 * a + 1]) : fabs(P.dx / sincos[2 * a]);
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    if (b < nb)
-                        proj[(static_cast<size_t>(b0 + b) * P.na + a) * P.ns + s] =
-                            static_cast<float>(static_cast<double>(sum[v][b]) * dw);
-            }
-        }
-    }
 }
 
 // Pixels of the image border (first / last row and column), i < 2nx + 2(ny-2).
@@ -467,78 +285,109 @@ int launch_fp(const FpProblem& P, const T* img, const T* imgT, T* proj, const do
     return check_launch("fp_kernel");
 }
 
-// Views per workgroup, at most kFpViews: 4 measured 0.78 ms on the
-// 8 x 512^2, 720-view scan, 2 0.89 ms (each staged row chunk serves half as
-// many rays) and, before the chunk pipeline, 8 1.26 ms (two waves per SIMD;
-// 178 VGPRs with it).  Small scans take fewer (fp_views) so that the grid
-// still fills the GPU.
-constexpr int kFpViews = 4;
-constexpr int kFpSlices = 4;
-// Two buffers of 2-row chunks with 512-column spans (32 KB of LDS at 4
-// slices; 97 VGPRs, four waves per SIMD): 0.775 ms on that scan, against
-// 0.84 ms for one buffer of 4-row chunks (no overlap of the DMAs with the
-// walk), 0.99 ms for two buffers of 4 rows (64 KB, two workgroups per CU),
-// 0.79 ms for two of 1 row and 0.88 ms with the VGPRs held to 95 for five
-// waves per SIMD.  Taking the taps of all V views branch-free (rays off the
-// image reading a zero pad) so their LDS reads overlap measured 0.84 ms:
-// whole waves then no longer skip the views they miss.  Staging rows of a
-// slice-interleaved copy (a ray step's taps of four slices in two
-// ds_read_b128 instead of four ds_read2st64_b32) measured 1.11 ms.
-constexpr int kFpRowsDefault = 2, kFpSpanDefault = 512;
-
-// Columns the rays of one fp_lds_kernel chunk can span: cpb channels at up
-// to sqrt(2) ds / pixel per channel, kFpRows rows at up to one column per row
-// (in pixel units of the marched axis), and the drift of a ray's column
-// across `views` views (at most 4 R |orbit| per view for an image of
-// half-diagonal R pixels), plus margins.
-bool fp_lds_applies(const ctr_geom& g, int views, int rows = kFpRowsDefault,
-                    int span_max = kFpSpanDefault)
+// Columns the rays of one fp_stream_kernel chunk can span: 64 channels at up to
+// sqrt(2) ds / pixel per channel, one column per further row, the drift of a ray
+// that is on the image across the other views (at most the image's
+// half-diagonal times sqrt(2) per radian, doubled for the second order), margins.
+bool fp_stream_applies(const ctr_geom& g, int views, int rows, int span_max)
 {
     const double pmin = std::min(std::fabs(g.dx), std::fabs(g.dy));
     const double pmax = std::max(std::fabs(g.dx), std::fabs(g.dy));
     if (!(pmin > 0) || !(g.ds > 0)) return false;
     const double r = 0.5 * std::hypot(g.nx + 2 * std::fabs(g.offset_x),
                                       g.ny + 2 * std::fabs(g.offset_y)) * pmax / pmin;
-    const int cpb = div_up(g.ns, div_up(g.ns, 256));  // channels per workgroup
-    const double span = (cpb - 1) * std::sqrt(2.0) * g.ds / pmin + rows * pmax / pmin +
-                        4.0 * r * views * std::fabs(g.orbit) + 8.0;
-    return span + 2.0 <= span_max;
+    const double turn = (views - 1) * std::fabs(g.orbit);
+    const double span = 63 * std::sqrt(2.0) * g.ds / pmin + (rows - 1) * pmax / pmin +
+                        1.5 * r * turn * (1.0 + 2.0 * turn) + 6.0;
+    // steps within 2 columns a row, one plane within a 31-bit buffer range
+    return span <= span_max && pmax <= 1.9 * pmin && 16LL * g.nx * g.ny < (1LL << 31);
 }
 
-// Views per workgroup for nb slices per workgroup: the most (up to
-// kFpViews) that leave at least 3 workgroups per CU (768 of the 1024 the
-// chip holds at four waves per SIMD), else 1.  On 8 x 512^2 images with
-// 729 channels, 640 to 680 views (960 to 1020 workgroups at 4 views) took
-// 0.73 ms at 4 views against 0.76-0.84 ms at 2, when the bar was 1024.
-int fp_views(const ctr_geom& g, int nbatch, int nb)
+// Waves (row segments) per workgroup: 2 where that fills the chip, more for small
+// scans (8 x 512^2, 720 views: 296 us at 2, 303 at 4, 345 at 8; 4 slices 184, 183,
+// 192; one slice 135, 120, 121; 1 x 256^2, 360 views: 68, 54, 54; 8 x 192^2, 200
+// views: 61, 55, 61).
+template <int NB, int V, int SPAN>
+int launch_fp_stream_s(FpStreamLaunch L, int n, hipStream_t st)
 {
-    const long long blocks = static_cast<long long>(div_up(g.ns, 256)) * div_up(nbatch, nb);
-    for (int v = kFpViews; v > 1; v /= 2)
-        if (blocks * div_up(g.na, v) >= 768) return v;
-    return 1;
+    using S = FpShape<NB, SPAN>;
+    L.nb = n;
+    L.cgroups = div_up(L.P.ns, 64);
+    const int groups = div_up(n, NB), vgroups = div_up(L.P.na, V);
+    const int steps = std::max(L.P.nx, L.P.ny);
+    const long long blocks = static_cast<long long>(L.cgroups) * vgroups * groups;
+    const int w = blocks >= 4096 ? 2 : 4;
+    L.chunks = div_up(div_up(steps, S::kRows), w);
+    const size_t lds = static_cast<size_t>(w) * S::kLds;
+    hipLaunchKernelGGL((fp_stream_kernel<NB, V, SPAN>), dim3(L.cgroups * vgroups, groups, 2),
+                       dim3(64 * w), lds, st, L);
+    return check_launch("fp_stream_kernel");
 }
 
-template <int NB, int V, int R = kFpRowsDefault, int SPAN = kFpSpanDefault>
-int launch_fp_lds(const FpProblem& P, const float* img, const float* imgT, float* proj,
-                  const double* sc, const double* bo, const int* usex, hipStream_t st)
-{
-    // channels split evenly over ceil(ns / 256) workgroups
-    const int nblk = div_up(P.ns, 256);
-    const int cpb = div_up(P.ns, nblk);
-    dim3 grid(nblk, div_up(P.na, V), div_up(P.nbatch, NB));
-    hipLaunchKernelGGL((fp_lds_kernel<NB, V, R, SPAN>), grid, dim3(256), 0, st, img, imgT, proj,
-                       sc, bo, usex, P, cpb);
-    return check_launch("fp_lds_kernel");
-}
-
+// shape: 0 4 views and 128 columns, 1 4 and 256, 2 1 and 128, 3 1 and 256.
 template <int NB>
-int launch_fp_lds_v(int views, const FpProblem& P, const float* img, const float* imgT,
-                    float* proj, const double* sc, const double* bo, const int* usex,
-                    hipStream_t st)
+int launch_fp_stream(int shape, const FpStreamLaunch& L, int n, hipStream_t st)
 {
-    return views >= 4 ? launch_fp_lds<NB, 4>(P, img, imgT, proj, sc, bo, usex, st)
-           : views >= 2 ? launch_fp_lds<NB, 2>(P, img, imgT, proj, sc, bo, usex, st)
-                        : launch_fp_lds<NB, 1>(P, img, imgT, proj, sc, bo, usex, st);
+    switch (shape) {
+        case 0: return launch_fp_stream_s<NB, 4, 128>(L, n, st);
+        case 1: return launch_fp_stream_s<NB, 4, 256>(L, n, st);
+        case 2: return launch_fp_stream_s<NB, 1, 128>(L, n, st);
+        default: return launch_fp_stream_s<NB, 1, 256>(L, n, st);
+    }
+}
+
+// Four views share a staged row unless their rays drift too far apart (few
+// views); 256 columns take coarse detectors.  -1: none.
+int fp_stream_shape(const ctr_geom& g)
+{
+    constexpr int rows = FpShape<1, 128>::kRows;
+    for (int shape = 0; shape < 4; ++shape)
+        if (fp_stream_applies(g, shape < 2 ? 4 : 1, rows, shape & 1 ? 256 : 128)) return shape;
+    return -1;
+}
+
+int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int nbatch, const double* sc,
+              const double* bo, const int* usex, hipStream_t st)
+{
+    FpStreamLaunch L{};
+    L.P = FpProblem{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
+                    static_cast<int>(g.ny), nbatch, g.dx, g.dy};
+    L.proj = proj;
+    L.sincos = sc;
+    L.bo = bo;
+    L.usex = usex;
+    const size_t slice = static_cast<size_t>(g.nx) * g.ny;
+    const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
+    const bool single = nbatch % 4 == 1;  // the last slice alone
+    float* ws = nullptr;
+    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&ws), (8 * np + (single ? 1 : 0)) * slice * sizeof(float), st));
+    float *rows = ws, *cols = ws + 4 * np * slice, *one = ws + 8 * np * slice;
+    const dim3 tiles(div_up(g.nx, 32), div_up(g.ny, 32), std::max(np, 1));
+    if (np)
+        hipLaunchKernelGGL(image_planes_kernel<4>, tiles, dim3(32, 8), 0, st, img, rows, cols,
+                           L.P.ny, L.P.nx, nbatch);
+    if (single)
+        hipLaunchKernelGGL(image_planes_kernel<1>, dim3(tiles.x, tiles.y), dim3(32, 8), 0, st,
+                           img + (nbatch - 1) * slice, nullptr, one, L.P.ny, L.P.nx, 1);
+    int rc = check_launch("image_planes_kernel");
+    for (int b0 = 0; b0 < nbatch && rc == CTR_OK;) {
+        const int left = nbatch - b0;
+        int take = left;
+        L.b0 = b0;
+        L.rows = rows;
+        L.cols = cols;
+        if (left >= 2) {
+            take = left % 4 == 1 ? left - 1 : left;
+            rc = launch_fp_stream<4>(shape, L, take, st);
+        } else {
+            L.rows = img;                   // indexed by slice
+            L.cols = one - b0 * slice;
+            rc = launch_fp_stream<1>(shape, L, 1, st);
+        }
+        b0 += take;
+    }
+    CTR_HIP(ctr::ws_free(ws, st));
+    return rc;
 }
 
 template <typename T>
@@ -547,6 +396,10 @@ int fp_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const double*
 {
     FpProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
                 static_cast<int>(g.ny), nbatch, g.dx, g.dy};
+    if constexpr (std::is_same<T, float>::value) {
+        const int shape = fp_stream_shape(g);
+        if (shape >= 0) return fp_stream(g, shape, img, proj, nbatch, sc, bo, usex, st);
+    }
     T* imgT = nullptr;
     const size_t n = static_cast<size_t>(nbatch) * g.nx * g.ny;
     CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&imgT), n * sizeof(T), st));
@@ -554,17 +407,6 @@ int fp_typed(const ctr_geom& g, const T* img, T* proj, int nbatch, const double*
                        dim3(32, 8), 0, st, img, imgT, static_cast<int>(g.ny),
                        static_cast<int>(g.nx));
     int rc = check_launch("transpose_kernel");
-    if constexpr (std::is_same<T, float>::value) {
-        const int nb = nbatch >= kFpSlices ? kFpSlices : nbatch >= 2 ? 2 : 1;
-        const int views = fp_views(g, nbatch, nb);
-        if (rc == CTR_OK && fp_lds_applies(g, views)) {
-            rc = nb == kFpSlices ? launch_fp_lds_v<kFpSlices>(views, P, img, imgT, proj, sc, bo, usex, st)
-                 : nb == 2       ? launch_fp_lds_v<2>(views, P, img, imgT, proj, sc, bo, usex, st)
-                                 : launch_fp_lds_v<1>(views, P, img, imgT, proj, sc, bo, usex, st);
-            CTR_HIP(ctr::ws_free(imgT, st));
-            return rc;
-        }
-    }
     if (rc == CTR_OK) {
         const int nb = nbatch >= 8 ? 8 : nbatch >= 4 ? 4 : nbatch >= 2 ? 2 : 1;
         switch (nb) {

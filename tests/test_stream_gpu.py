@@ -164,3 +164,42 @@ def test_workspace_is_given_back(F):
     torch.cuda.synchronize()
     _lib.call("ctr_release_workspace")
     assert torch.equal(a, F.fan_backprojection_2d(x, **kwargs(g, True)))
+
+
+# (nx, ny, views, channels, ds, slices, orbit_start): partial row segments and
+# chunks, groups with views of both branches, rays that run along an image edge
+# or cross a pixel corner exactly (odd sizes, no offsets), few views (one per
+# workgroup), coarse detectors (256 staged columns, and beyond: the FP64-position
+# kernel), detectors narrower and wider than the image
+FP = [(33, 33, 40, 47, 1.0, 1, 0.0), (33, 33, 40, 47, 1.0, 5, 0.0), (32, 32, 40, 47, 1.0, 4, 0.0),
+      (64, 48, 37, 80, 1.0, 2, 0.1), (48, 64, 37, 80, 1.0, 3, -0.7), (5, 3, 9, 12, 1.0, 1, 0.0),
+      (3, 70, 22, 90, 0.8, 4, 0.3), (130, 130, 6, 150, 1.0, 1, 0.05), (130, 130, 6, 150, 1.0, 6, 0.05),
+      (90, 90, 45, 70, 2.0, 1, 0.2), (90, 90, 45, 70, 2.0, 4, 0.2), (90, 90, 45, 30, 4.5, 2, 0.2),
+      (200, 200, 50, 41, 1.0, 1, 0.0), (65, 65, 72, 200, 0.7071067811865476, 9, 0.0),
+      (257, 255, 16, 257, 1.0, 1, 0.7853981633974483)]
+
+
+@pytest.mark.parametrize("case", range(len(FP)))
+@pytest.mark.parametrize("offset", [0.0, 0.3])
+def test_fp_stream_matches_oracle(F, case, offset):
+    nx, ny, na, ns, ds, n, start = FP[case]
+    g = dict(nx=nx, ny=ny, na=na, ns=ns, dx=1.0, dy=1.0, ds=ds, offset_x=offset, offset_y=-offset,
+             offset_s=offset, orbit_start=start, orbit=math.pi / na)
+    og = O.geom(**g)
+    t = O.fp_prep(og)
+    img = randn(1000 + case, (n, ny, nx))
+    out = F.parallel_projection_2d(torch.from_numpy(img).cuda(), **kwargs(g, False)).cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.fp(og, img[b], t)) < TOL32, b
+
+
+@pytest.mark.parametrize("n", [1, 4])
+def test_fp_nonfinite_pixels_stay_in_their_rays(F, n):
+    g = geom(40, 30, 60, 1.0, 1.0, fan=False)
+    img = randn(1100, (n, 40, 40))
+    img[0, 0, 39], img[0, 20, 11], img[n - 1, 39, 0] = np.inf, np.nan, -np.inf
+    og = O.geom(**g)
+    t = O.fp_prep(og)
+    out = F.parallel_projection_2d(torch.from_numpy(img).cuda(), **kwargs(g, False)).cpu().numpy()
+    for b in range(n):
+        np.testing.assert_array_equal(np.isfinite(out[b]), np.isfinite(O.fp(og, img[b], t)))
