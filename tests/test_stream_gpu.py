@@ -203,3 +203,22 @@ def test_fp_nonfinite_pixels_stay_in_their_rays(F, n):
     out = F.parallel_projection_2d(torch.from_numpy(img).cuda(), **kwargs(g, False)).cpu().numpy()
     for b in range(n):
         np.testing.assert_array_equal(np.isfinite(out[b]), np.isfinite(O.fp(og, img[b], t)))
+
+
+# distance-driven pair on interleaved planes, bitwise: group sizes 8 and 4 and
+# their remainders, footprints of one, two and many cells (and channels), spans
+# and footprints cut by the image's and the detector's ends
+@pytest.mark.parametrize("n", [1, 4, 5, 9])
+@pytest.mark.parametrize("ds,ns,na", [(1.0, 51, 24), (0.3, 60, 9), (4.5, 14, 16), (1.0, 9, 8)])
+def test_dd_planes_match_oracle_bitwise(F, n, ds, ns, na):
+    g = geom(35, na, ns, 1.0, ds, fan=False, offset_s=0.0)
+    g.update(offset_x=0.0, offset_y=0.0, orbit_start=0.0)
+    og = O.geom(**g)
+    img, proj = randn(1200 + n, (n, 35, 35)), randn(1210 + n, (n, na, ns))
+    kw = kwargs(g, False)
+    fp = F.parallel_projection_2d(torch.from_numpy(img).cuda(), method="disdriven", **kw)
+    gr = F.parallel_projection_2d_grad(torch.from_numpy(proj).cuda(), method="disdriven", **kw)
+    t, tg = O.fp_dd_prep(og), O.fp_dd_grad_prep(og)
+    for b in range(n):
+        np.testing.assert_array_equal(fp[b].cpu().numpy(), O.fp_dd(og, img[b], t))
+        np.testing.assert_array_equal(gr[b].cpu().numpy(), O.fp_dd_grad(og, proj[b], tg))
