@@ -1,14 +1,19 @@
 // Device memory the operators need only during a call (transposed copies,
-// interleaved sinograms, partial sums): stream-ordered allocations from one
-// pool per device.
+// interleaved sinograms, partial sums).
 //
-// The device's default pool gives everything back whenever a stream is
-// synchronised, so a program that waits for each result paid for mapping the
-// memory again on every call (about 100 us for the ray-driven FP and its
-// transpose, 150 us of the 1.2 ms of a least-squares gradient).  This pool
-// keeps up to kKeep bytes that are free, no more, and ctr_release_workspace
-// gives those back too.  The pool orders reuse between streams itself and is
-// safe to use from several threads.
+// A stream-ordered allocation and its release cost the host 15 to 25 us a call
+// once kernels lie between the two, as much as the rest of a small operator,
+// and the default pool maps the memory anew after every synchronisation (about
+// 100 us).  So freed blocks are kept, per device, with an event recorded where
+// their last use ends: a call on the same stream takes one at once (the wait
+// for the event is then satisfied by the stream's order), a call on another
+// stream only a block whose event has passed.  At most kKeep bytes and
+// kBlocks blocks are kept free, the oldest go first, and ctr_release_workspace
+// gives them all back.  Any number of threads and streams: a block belongs to
+// one call from ws_alloc to ws_free.
+#include <cstdint>
+#include <deque>
+#include <exception>
 #include <mutex>
 #include <unordered_map>
 
@@ -19,55 +24,123 @@ namespace {
 
 // 1 GiB: the scratch of the largest sinogram batch of the benchmark (32 x 1440
 // x 1472) four times over
-constexpr uint64_t kKeep = 1ull << 30;
+constexpr size_t kKeep = size_t{1} << 30, kBlocks = 64;
+
+struct Block {
+    void* p;
+    size_t bytes;
+    hipEvent_t done;  // recorded after the last use
+    hipStream_t st;   // stream of the last use
+};
+
+struct Device {
+    std::deque<Block> free;  // oldest first
+    size_t free_bytes = 0;
+};
 
 std::mutex g_mu;
-std::unordered_map<int, hipMemPool_t> g_pools;  // device -> pool, for the process's life
+std::unordered_map<int, Device> g_devices;
+std::unordered_map<void*, Block> g_used;  // blocks a call holds
 
-hipError_t pool_of_device(hipMemPool_t* out)
+// Blocks come in sizes of 1/4 octave, so that calls of similar sizes share them.
+size_t block_size(size_t bytes)
 {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(g_mu);
-    auto it = g_pools.find(dev);
-    if (it == g_pools.end()) {
-        hipMemPoolProps props{};
-        props.allocType = hipMemAllocationTypePinned;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        hipMemPool_t pool = nullptr;
-        e = hipMemPoolCreate(&pool, &props);
-        if (e != hipSuccess) return e;
-        uint64_t keep = kKeep;
-        e = hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-        if (e != hipSuccess) {
-            (void)hipMemPoolDestroy(pool);
-            return e;
-        }
-        it = g_pools.emplace(dev, pool).first;
+    size_t step = size_t{1} << 16;
+    while (step * 8 <= bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
     }
-    *out = it->second;
-    return hipSuccess;
+    return status != hipStreamCaptureStatusNone;
 }
 
 }  // namespace
 
 hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
 {
-    // a captured allocation belongs to the graph, which has a pool of its own
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return hipMallocAsync(p, bytes, st);
+    // a captured allocation belongs to the graph, which has memory of its own
+    if (capturing(st)) return hipMallocAsync(p, bytes, st);
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const size_t want = block_size(bytes);
+    try {
+        std::lock_guard<std::mutex> lock(g_mu);
+        Device& D = g_devices[dev];
+        // newest first: its lines may still be in the caches
+        for (size_t i = D.free.size(); i-- > 0;) {
+            Block b = D.free[i];
+            if (b.bytes < bytes || b.bytes > 2 * want) continue;
+            if (b.st != st && hipEventQuery(b.done) != hipSuccess) {
+                (void)hipGetLastError();  // not ready
+                continue;
+            }
+            // (a destroyed stream's handle may name a new stream: hence the wait)
+            e = hipStreamWaitEvent(st, b.done, 0);
+            if (e != hipSuccess) return e;
+            g_used.emplace(b.p, b);
+            D.free.erase(D.free.begin() + static_cast<std::ptrdiff_t>(i));
+            D.free_bytes -= b.bytes;
+            *p = b.p;
+            return hipSuccess;
+        }
+        Block b{nullptr, want, nullptr, st};
+        e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming);
+        if (e != hipSuccess) return e;
+        e = hipMallocAsync(&b.p, want, st);
+        if (e == hipSuccess) {
+            g_used.emplace(b.p, b);
+            *p = b.p;
+        } else {
+            (void)hipEventDestroy(b.done);
+        }
+        return e;
+    } catch (const std::exception&) {
+        return hipErrorOutOfMemory;
     }
-    if (status != hipStreamCaptureStatusNone) return hipMallocAsync(p, bytes, st);
-    hipMemPool_t pool = nullptr;
-    const hipError_t e = pool_of_device(&pool);
-    return e == hipSuccess ? hipMallocFromPoolAsync(p, bytes, pool, st) : e;
 }
 
-hipError_t ws_free(void* p, hipStream_t st) { return hipFreeAsync(p, st); }
+hipError_t ws_free(void* p, hipStream_t st)
+{
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    try {
+        std::lock_guard<std::mutex> lock(g_mu);
+        const auto it = g_used.find(p);
+        if (it == g_used.end()) return hipFreeAsync(p, st);  // a captured allocation
+        Block b = it->second;
+        g_used.erase(it);
+        b.st = st;
+        e = hipEventRecord(b.done, st);
+        if (e != hipSuccess) {
+            (void)hipEventDestroy(b.done);
+            const hipError_t f = hipFreeAsync(p, st);
+            return f != hipSuccess ? f : e;
+        }
+        Device& D = g_devices[dev];
+        D.free.push_back(b);
+        D.free_bytes += b.bytes;
+        while (D.free_bytes > kKeep || D.free.size() > kBlocks) {
+            const Block old = D.free.front();
+            D.free.pop_front();
+            D.free_bytes -= old.bytes;
+            e = hipStreamWaitEvent(st, old.done, 0);
+            if (e == hipSuccess) e = hipFreeAsync(old.p, st);
+            (void)hipEventDestroy(old.done);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    } catch (const std::exception&) {
+        return hipErrorOutOfMemory;
+    }
+}
 
 }  // namespace ctr
 
@@ -76,10 +149,20 @@ extern "C" int ctr_release_workspace(void)
     using namespace ctr;
     try {
         std::lock_guard<std::mutex> lock(g_mu);
-        for (auto& entry : g_pools) CTR_HIP(hipMemPoolTrimTo(entry.second, 0));
+        int dev = 0;
+        CTR_HIP(hipGetDevice(&dev));
+        Device& D = g_devices[dev];
+        while (!D.free.empty()) {
+            const Block b = D.free.back();
+            D.free.pop_back();
+            D.free_bytes -= b.bytes;
+            CTR_HIP(hipEventSynchronize(b.done));
+            (void)hipEventDestroy(b.done);
+            CTR_HIP(hipFree(b.p));
+        }
         return CTR_OK;
-    } catch (...) {
-        set_error("ctr_release_workspace: out of memory");
+    } catch (const std::exception& e) {
+        set_error(std::string("ctr_release_workspace: ") + e.what());
         return CTR_ERR_ALLOC;
     }
 }

@@ -61,8 +61,8 @@ typedef struct ctr_geom {
 const char* ctr_last_error(void);
 /* Library version as 10000*major + 100*minor + patch. */
 int ctr_version(void);
-/* Operators take scratch memory from one stream-ordered pool per device, which
- * keeps up to 1 GiB of it between calls; this gives the free part back. */
+/* Operators keep up to 1 GiB of scratch memory per device between calls; this
+ * waits for its last uses and gives the current device's back. */
 int ctr_release_workspace(void);
 /* Device properties the kernels are tuned on (for reports). */
 int ctr_device_info(int* cu_count, int* clock_khz, int* lds_bytes_per_cu, char* arch,

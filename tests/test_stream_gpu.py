@@ -222,3 +222,53 @@ def test_dd_planes_match_oracle_bitwise(F, n, ds, ns, na):
     for b in range(n):
         np.testing.assert_array_equal(fp[b].cpu().numpy(), O.fp_dd(og, img[b], t))
         np.testing.assert_array_equal(gr[b].cpu().numpy(), O.fp_dd_grad(og, proj[b], tg))
+
+
+def test_workspace_across_streams_and_threads(F):
+    """Calls that need scratch, from several streams and threads at once and
+    with changing sizes, give the results of calls one after the other."""
+    import threading
+    cases = [(geom(40 + 8 * k, 30 + k, 60 + 10 * k, 1.0, 1.0, fan=False), 1 + k % 5)
+             for k in range(6)]
+    xs = [torch.from_numpy(randn(1300 + k, (n, g["ny"], g["nx"]))).cuda()
+          for k, (g, n) in enumerate(cases)]
+    want = [F.parallel_projection_2d(x, **kwargs(g, False)) for x, (g, _) in zip(xs, cases)]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(seed):
+        st = torch.cuda.Stream()
+        rng = np.random.default_rng(seed)
+        with torch.cuda.stream(st):
+            got = [(k, F.parallel_projection_2d(xs[k], **kwargs(cases[k][0], False)))
+                   for k in rng.integers(0, len(cases), 60)]
+        st.synchronize()
+        bad.extend(k for k, y in got if not torch.equal(y, want[k]))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
+
+
+def test_captured_call_replays(F):
+    """A captured call takes its scratch from the graph: replays with new
+    inputs, eager work on other sizes in between."""
+    g = geom(48, 40, 70, 1.0, 1.0, fan=False)
+    kw = kwargs(g, False)
+    x = torch.from_numpy(randn(1400, (4, 48, 48))).cuda()
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        F.parallel_projection_2d(x, **kw)
+    torch.cuda.current_stream().wait_stream(st)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = F.parallel_projection_2d(x, **kw)
+    for k in range(4):
+        x.copy_(torch.from_numpy(randn(1401 + k, (4, 48, 48))))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = y.clone()
+        assert torch.equal(got, F.parallel_projection_2d(x, **kw)), k
+        F.parallel_projection_2d(x[:2], **kw)
