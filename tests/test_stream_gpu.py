@@ -272,3 +272,30 @@ def test_captured_call_replays(F):
         got = y.clone()
         assert torch.equal(got, F.parallel_projection_2d(x, **kw)), k
         F.parallel_projection_2d(x[:2], **kw)
+
+
+FAN64 = [
+    (geom(64, 90, 96, 0.7, 1.3), 1), (geom(50, 45, 80, 0.7, 1.3, ny=37), 2),
+    (geom(33, 61, 70, 0.7, 1.3), 3), (geom(17, 129, 40, 0.7, 1.3), 4),  # rounds of 128 views
+    (geom(7, 257, 40, 0.7, 1.3), 7), (geom(96, 60, 41, 0.7, 1.3, offset_s=11.0), 5),
+    (geom(40, 1, 64, 0.7, 1.3), 2), (geom(40, 20, 2, 0.7, 300.0, offset_s=0.1), 2),
+    (geom(32, 50, 64, 6.0, 2.0), 3),  # |u| above 0.1: the plain kernel
+    # pixels exactly at the first and at the last channel of the first view
+    (dict(geom(33, 8, 32, 1.0, 1.3, offset_s=-15.5), offset_x=0.0, orbit_start=0.0), 1),
+    (dict(geom(33, 8, 32, 1.0, 1.3, offset_s=15.5), offset_x=0.0, orbit_start=0.0), 2),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FAN64)))
+def test_fan_bp_float64_matches_oracle(F, case):
+    """Tile anchors in FP64: positions are the reference's to a few 1e-13 channel
+    (the rounding of s, |s| < 1e3, and of its offset), so 1e-12 relative L2."""
+    g, n = FAN64[case]
+    og = O.geom(**g)
+    t = O.fan_prep(og)
+    proj = np.random.default_rng(1100 + case).standard_normal((n, g["na"], g["ns"]))
+    out = F.fan_backprojection_2d(torch.from_numpy(proj).cuda(), **kwargs(g, True))
+    assert out.dtype == torch.float64
+    out = out.cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.fan_bp(og, proj[b], t)) < 1e-12, b
