@@ -299,3 +299,14 @@ def test_fan_bp_float64_matches_oracle(F, case):
     out = out.cpu().numpy()
     for b in range(n):
         assert rel_l2(out[b], O.fan_bp(og, proj[b], t)) < 1e-12, b
+
+
+@pytest.mark.parametrize("ns", [2, 3, 8, 15, 16, 17, 31, 255, 256, 257, 513, 1025, 1706])
+def test_ramp_float64_matches_oracle(F, ns):
+    """Rows around a lane's 4 outputs, a block's 8 samples, the near field's 15 taps
+    and a wave's 256 outputs, up to the longest; sums of at most 853 FP64 products,
+    so 1e-12 relative L2."""
+    g = O.geom(ns=ns, nrow=5, ds=0.9, dsd=1085.6, type=1)
+    x = np.random.default_rng(1200 + ns).standard_normal((5, ns))
+    out = F.ramp_filter(torch.from_numpy(x).cuda(), ns, 5, 0.9, 1085.6, "fan").cpu().numpy()
+    assert rel_l2(out, O.ramp(g, x, O.ramp_prep(g))) < 1e-12
