@@ -1,9 +1,8 @@
 // Forward backprojection with wave-private view streams (float32), for the
 // geometries whose detector position is a low-order polynomial along a short
-// run of pixels.  It serves every slice count the 16-slice engine kernel
-// (bp_engine.hpp) does not: there the geometry of a pixel-view is shared by
-// 16 slices, here by 8, 4, 2 or 1, so what bounds the kernel is the issue of
-// that geometry, and the work is split to make it cheap:
+// run of pixels (others: bp_engine.hpp).  What bounds a BP is the issue of the
+// geometry of a pixel-view, the more so the fewer slices (16, 8, 4, 2 or 1) share
+// it, and the work is split to make it cheap:
 //  * a lane owns a run of M pixels of an image row.  Per view it evaluates
 //    the geometry once, at the run's centre, with its derivatives along the
 //    row (Geo::run), and every pixel of the run takes the position and the
@@ -551,7 +550,7 @@ inline bool stream_applies(int lmax, long long na, long long ns)
 // slices included: 10 to 15 slices are one group of 16 (8 + 4: 340), 5 to 7 one
 // of 8 (4 + 1: 224), 3 one of 4.  RAW: nothing is allocated.
 template <class Geo, bool RAW = false>
-int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, const float* proj,
+int launch_stream_part(StreamLaunch<Geo> L, const typename Geo::Tables& T, const float* proj,
                         int n, int lmax, hipStream_t st)
 {
     const auto& P = L.P;
@@ -561,7 +560,8 @@ int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, cons
     float* ws = nullptr;
     if (n > 1 && !RAW) {
         const size_t slices = n == 2 ? 2 : div_up(n, 4) * 4;
-        CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&ws), slices * sino * sizeof(float), st));
+        const int e = ws_part(reinterpret_cast<void**>(&ws), slices * sino * sizeof(float), n, st);
+        if (e) return e;
         const dim3 grid(div_up(sino, 256), n == 2 ? 1 : div_up(n, 4));
         if (n == 2)
             hipLaunchKernelGGL(interleave_kernel<2>, grid, dim3(256), 0, st, proj, ws,
@@ -594,6 +594,20 @@ int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, cons
     }
     if (ws) CTR_HIP(ctr::ws_free(ws, st));
     return rc;
+}
+
+template <class Geo, bool RAW = false>
+int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, const float* proj,
+                        int n, int lmax, hipStream_t st)
+{
+    if (RAW) return launch_stream_part<Geo, true>(L, T, proj, n, lmax, st);
+    const size_t sino = static_cast<size_t>(L.P.na) * L.P.ns;
+    const size_t image = static_cast<size_t>(L.P.nx) * L.P.ny;
+    float* const img = L.img;
+    return in_parts(n, sino * sizeof(float), [&](int b, int count) {
+        L.img = img + b * image;
+        return launch_stream_part<Geo>(L, T, proj + b * sino, count, lmax, st);
+    });
 }
 
 }  // namespace ctr

@@ -56,6 +56,38 @@ inline double cent_s(const ctr_geom& g) { return static_cast<double>(g.ns - 1) /
 hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st);
 hipError_t ws_free(void* p, hipStream_t st);
 
+// A batch in parts whose scratch (bytes a slice) stays within 1 GiB, at least 16
+// slices each: call(first, count).  A part whose scratch the device has no room for
+// (ws_part: kNoScratch) is called slice by slice, which needs next to none.
+constexpr int kNoScratch = -1;
+
+inline int ws_part(void** p, size_t bytes, int count, hipStream_t st)
+{
+    const hipError_t e = ws_alloc(p, bytes, st);
+    if (e == hipErrorOutOfMemory && count > 1) {
+        (void)hipGetLastError();
+        return kNoScratch;
+    }
+    CTR_HIP(e);
+    return 0;
+}
+
+template <typename F>
+int in_parts(int n, size_t bytes, F&& call)
+{
+    const size_t fit = (size_t{1} << 30) / bytes / 16 * 16;
+    const int part = static_cast<int>(fit < 16 ? 16 : fit < static_cast<size_t>(n) ? fit : n);
+    int rc = 0;
+    for (int b = 0; b < n && rc == 0; b += part) {
+        const int count = n - b < part ? n - b : part;
+        rc = call(b, count);
+        if (rc != kNoScratch) continue;
+        rc = 0;
+        for (int i = 0; i < count && rc == 0; ++i) rc = call(b + i, 1);
+    }
+    return rc;
+}
+
 // Scale of bp_fan_2d: |orbit| / round(|na*orbit|/pi) (src/bp_fan_2d.cc:58,83).
 double fan_bp_scale(const ctr_geom& g);
 

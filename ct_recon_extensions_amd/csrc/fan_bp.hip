@@ -1,11 +1,11 @@
 // Fan-beam pixel-driven backprojection for gfx950 (bp_fan_2d and
 // bp_fan_2d_angle), its exact transpose, and the reference-structured
-// baseline.  The forward kernel and the transpose are the BP engine
-// (bp_engine.hpp) with the fan geometry policy (fan_geom.hpp): workgroups of
-// one pixel tile x NB slices sharing the geometry, LDS-staged detector spans,
-// FP64 per-(tile, view) anchors and FP32 pixel offsets; the transpose gathers
-// each (view, channel) output in registers from the pixels that reach it
-// (bp_gather.hpp), with the forward's anchors and pixel geometry.
+// baseline.  float32: FP64 anchors per (tile, view) and FP32 offsets, on runs of
+// pixels (bp_stream.hpp) where the geometry is a low-order polynomial along them
+// (fan_run_order), else pixel by pixel (bp_engine.hpp); float64: the same anchors
+// with FP64 offsets (fan_bp_f64_kernel).  The transpose gathers each (view,
+// channel) output in registers from the pixels that reach it (bp_gather.hpp), with
+// the pixel geometry of fan_geom.hpp.
 //
 // Edge rule (src/bp_fan_2d.cc:72-80): a pixel-view contributes iff
 // 0 <= s <= ns-1, with taps floor(s) and ceil(s).

@@ -528,7 +528,7 @@ int dd_groups(int nbatch, F&& launch)
     return CTR_OK;
 }
 
-int fp_dd_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, const double* sc,
+int fp_dd_f32_part(const ctr_geom& g, const float* img, float* proj, int nbatch, const double* sc,
               const double* bo, const int* usex, hipStream_t st)
 {
     DdProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
@@ -537,8 +537,9 @@ int fp_dd_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, cons
     const bool single = nbatch % 8 == 1;  // a last slice alone
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     float* ws = nullptr;
-    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&ws),
-                          (8 * np + (single ? 2 : 0)) * slice * sizeof(float), st));
+    const int e = ws_part(reinterpret_cast<void**>(&ws),
+                          (8 * np + (single ? 2 : 0)) * slice * sizeof(float), nbatch, st);
+    if (e) return e;
     float *rows = ws, *cols = ws + 4 * np * slice, *one = ws + 8 * np * slice;
     const dim3 tiles(div_up(g.nx, 32), div_up(g.ny, 32)), block(32, 8);
     if (np)
@@ -569,7 +570,7 @@ int fp_dd_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, cons
     return rc;
 }
 
-int fp_dd_grad_f32(const ctr_geom& g, const float* proj, float* img, int nbatch, const double* w,
+int fp_dd_grad_f32_part(const ctr_geom& g, const float* proj, float* img, int nbatch, const double* w,
                    const double* pos, const int* usex, int stride, hipStream_t st)
 {
     DdProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
@@ -578,7 +579,8 @@ int fp_dd_grad_f32(const ctr_geom& g, const float* proj, float* img, int nbatch,
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     float* ws = nullptr;
     if (np) {
-        CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&ws), 4 * np * sino * sizeof(float), st));
+        const int e = ws_part(reinterpret_cast<void**>(&ws), 4 * np * sino * sizeof(float), nbatch, st);
+        if (e) return e;
         hipLaunchKernelGGL(interleave_kernel<4>, dim3(div_up(sino, 256), np), dim3(256), 0, st,
                            proj, ws, static_cast<unsigned int>(sino), nbatch);
     }
@@ -601,6 +603,25 @@ int fp_dd_grad_f32(const ctr_geom& g, const float* proj, float* img, int nbatch,
         });
     if (ws) CTR_HIP(ctr::ws_free(ws, st));
     return rc;
+}
+
+int fp_dd_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, const double* sc,
+              const double* bo, const int* usex, hipStream_t st)
+{
+    const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
+    return in_parts(nbatch, 2 * slice * sizeof(float), [&](int b, int count) {
+        return fp_dd_f32_part(g, img + b * slice, proj + b * sino, count, sc, bo, usex, st);
+    });
+}
+
+int fp_dd_grad_f32(const ctr_geom& g, const float* proj, float* img, int nbatch, const double* w,
+                   const double* pos, const int* usex, int stride, hipStream_t st)
+{
+    const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
+    return in_parts(nbatch, sino * sizeof(float), [&](int b, int count) {
+        return fp_dd_grad_f32_part(g, proj + b * sino, img + b * slice, count, w, pos, usex, stride,
+                                   st);
+    });
 }
 
 template <typename T, int NB>

@@ -346,7 +346,7 @@ int fp_stream_shape(const ctr_geom& g)
     return -1;
 }
 
-int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int nbatch, const double* sc,
+int fp_stream_part(const ctr_geom& g, int shape, const float* img, float* proj, int nbatch, const double* sc,
               const double* bo, const int* usex, hipStream_t st)
 {
     FpStreamLaunch L{};
@@ -360,7 +360,9 @@ int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int n
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     const bool single = nbatch % 4 == 1;  // the last slice alone
     float* ws = nullptr;
-    CTR_HIP(ctr::ws_alloc(reinterpret_cast<void**>(&ws), (8 * np + (single ? 1 : 0)) * slice * sizeof(float), st));
+    const int e = ws_part(reinterpret_cast<void**>(&ws),
+                          (8 * np + (single ? 1 : 0)) * slice * sizeof(float), nbatch, st);
+    if (e) return e;
     float *rows = ws, *cols = ws + 4 * np * slice, *one = ws + 8 * np * slice;
     const dim3 tiles(div_up(g.nx, 32), div_up(g.ny, 32), std::max(np, 1));
     if (np)
@@ -388,6 +390,15 @@ int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int n
     }
     CTR_HIP(ctr::ws_free(ws, st));
     return rc;
+}
+
+int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int nbatch,
+              const double* sc, const double* bo, const int* usex, hipStream_t st)
+{
+    const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
+    return in_parts(nbatch, 2 * slice * sizeof(float), [&](int b, int count) {
+        return fp_stream_part(g, shape, img + b * slice, proj + b * sino, count, sc, bo, usex, st);
+    });
 }
 
 template <typename T>

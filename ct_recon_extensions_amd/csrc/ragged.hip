@@ -6,10 +6,11 @@
 // ordered by cost (views x tile pixels, exact-mode tiles weighted up), and a
 // grid of exactly as many workgroups as the chip holds at once pulls items
 // from a global counter: longest-first list scheduling, so the tail is one
-// small item long.  Each item runs the shared tile engine (bp_engine.hpp)
-// with the problem's own span width and series/exact policy, picked per item
-// by a uniform branch; the tile shape and the views per LDS round are
-// launch-wide and come from the autotuner.
+// small item long.  Each 16 x 16 tile runs the view streams of bp_stream.hpp
+// where the problem's geometry allows (fan_run_order), any other the shared tile
+// engine (bp_engine.hpp) with the problem's own span width and series/exact
+// policy, picked per item by a uniform branch; the tile shape and the views per
+// LDS round are launch-wide and come from the autotuner.
 //
 // The counter is cleared by a one-thread kernel launched just before the
 // persistent kernel (no memset node), so the pair can be captured into a

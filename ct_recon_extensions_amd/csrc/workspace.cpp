@@ -94,6 +94,16 @@ hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
         e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming);
         if (e != hipSuccess) return e;
         e = hipMallocAsync(&b.p, want, st);
+        if (e == hipErrorOutOfMemory && !D.free.empty()) {  // the kept blocks make room
+            (void)hipGetLastError();
+            for (const Block& old : D.free) {
+                if (hipStreamWaitEvent(st, old.done, 0) == hipSuccess) (void)hipFreeAsync(old.p, st);
+                (void)hipEventDestroy(old.done);
+            }
+            D.free.clear();
+            D.free_bytes = 0;
+            e = hipMallocAsync(&b.p, want, st);
+        }
         if (e == hipSuccess) {
             g_used.emplace(b.p, b);
             *p = b.p;

@@ -310,3 +310,28 @@ def test_ramp_float64_matches_oracle(F, ns):
     x = np.random.default_rng(1200 + ns).standard_normal((5, ns))
     out = F.ramp_filter(torch.from_numpy(x).cuda(), ns, 5, 0.9, 1085.6, "fan").cpu().numpy()
     assert rel_l2(out, O.ramp(g, x, O.ramp_prep(g))) < 1e-12
+
+
+@pytest.mark.parametrize("op", ["fan", "fp", "dd", "dd_grad"])
+def test_batches_whose_scratch_comes_in_parts(F, op):
+    """18 slices of 64 MiB: the scratch of 16 at a time; the last two equal a call of
+    their own, bit for bit."""
+    torch.manual_seed(7)
+    if op == "fan":
+        g = geom(16, 1500, 11185, 0.7, 1.3)
+        x = torch.randn((18, 1500, 11185), device="cuda")
+        call = lambda x: F.fan_backprojection_2d(x, **kwargs(g, True))
+    else:
+        g = geom(4096 if op != "dd_grad" else 24, 4 if op != "dd_grad" else 1500,
+                 64 if op != "dd_grad" else 11185, 1.0, 1.0, fan=False)
+        kw = kwargs(g, False)
+        size = (4096, 4096) if op != "dd_grad" else (1500, 11185)
+        x = torch.randn((18, *size), device="cuda")
+        if op == "dd_grad":
+            call = lambda x: F.parallel_projection_2d_grad(x, method="disdriven", **kw)
+        else:
+            method = "disdriven" if op == "dd" else "raydriven"
+            call = lambda x: F.parallel_projection_2d(x, method=method, **kw)
+    out = call(x)
+    assert torch.equal(out[16:], call(x[16:]))
+    assert torch.equal(out[:16], call(x[:16]))
