@@ -46,6 +46,9 @@ PEAK_VALU_SLOTS = CU * LANES * CLK  # FP32 VALU lane-issues per second (3.93e13)
 # Per slice: two FMAs into the accumulator = 2.
 FAN_GEOM_SLOTS = 24
 FAN_SLICE_SLOTS = 2
+# The forward BP evaluates that geometry once per run of 8 pixels, with its
+# derivatives (43 slots), and each pixel from the run's polynomial (3.5).
+FAN_RUN_SLOTS = 9
 # Per-slice model with no geometry sharing (atan2 + divide per pixel*view,
 # the textbook count for one slice at a time).
 UNBATCHED_FAN_SLOTS = 28
@@ -281,8 +284,8 @@ def kw_dd():
 # on this workload (SQ_INSTS_VALU, profiles/fp_dd_8x512sq_720v_729ch.md).
 # The reference's float/double mix and operation order are kept for bit
 # identity, so issue, not HBM, bounds both kernels.
-DD_VALU_FP = 1.21e9
-DD_VALU_GRAD = 9.97e8
+DD_VALU_FP = 4.92e8
+DD_VALU_GRAD = 4.31e8
 
 
 def _dd_roofline(kernel, valu_insts, alg_bytes, ms):
@@ -339,8 +342,8 @@ def bench_fp_dd(torch, F, reps, with_cpu=True):
     res = {"workload": "8 x 512^2, parallel 720 views/180deg, 729 ch, ds=dx=1, distance-driven; "
                        "seeded N(0,1) image and sinogram", "seed": DD_SEED,
            "fp_ms": round(ms_fp, 4), "grad_ms": round(ms_gr, 4),
-           "roofline_fp": _dd_roofline("fp_dd_kernel", DD_VALU_FP, alg_fp, ms_fp),
-           "roofline_grad": _dd_roofline("fp_dd_grad_kernel", DD_VALU_GRAD, alg_gr, ms_gr)}
+           "roofline_fp": _dd_roofline("fp_dd_cells_kernel<8>", DD_VALU_FP, alg_fp, ms_fp),
+           "roofline_grad": _dd_roofline("fp_dd_grad_planes_kernel<8>", DD_VALU_GRAD, alg_gr, ms_gr)}
     if with_cpu:
         from oracle import oracle as O
         kind = "ref" if O.have_ref() else "oracle"
@@ -485,12 +488,12 @@ def bench_lsq(torch, steps):
         "fp_ray_samples_per_s": 8 * scan.na * scan.ns * scan.n / (ms_fp * 1e-3),
         "fpt_pixel_views_per_s": 8 * scan.na * scan.n ** 2 / (ms_fpt * 1e-3),
         "roofline_fp": _valu_roofline(
-            "fp_lds_kernel", 8 * scan.na * scan.ns * scan.n,
+            "fp_stream_kernel", 8 * scan.na * scan.ns * scan.n,
             FP_GEOM_SLOTS / FP_SLICES_PER_WG + FP_SLICE_SLOTS, ms_fp,
             f"ray sample ({FP_GEOM_SLOTS} per ray-row shared by {FP_SLICES_PER_WG} slices "
             f"+ {FP_SLICE_SLOTS} per slice)"),
         "roofline_fpt": _valu_roofline(
-            "bp_forward_kernel<FptGeo> + border passes", 8 * scan.na * scan.n ** 2,
+            "bp_stream_kernel<FptGeo> + border passes", 8 * scan.na * scan.n ** 2,
             FPT_GEOM_SLOTS / FPT_SLICES_PER_WG + FPT_SLICE_SLOTS, ms_fpt,
             f"pixel*view*slice ({FPT_GEOM_SLOTS} per pixel*view shared by "
             f"{FPT_SLICES_PER_WG} slices + {FPT_SLICE_SLOTS} per slice)"),
@@ -530,7 +533,7 @@ def bench_ragged(torch, reps):
             rb.pixel_views / (ms * 1e-3) * UNBATCHED_FAN_SLOTS / PEAK_VALU_SLOTS, 4),
         # one slice per problem: the geometry of every pixel*view is its own
         "roofline": _valu_roofline("ragged_fan_bp_kernel", rb.pixel_views,
-                                   FAN_GEOM_SLOTS + FAN_SLICE_SLOTS, ms, "pixel*view"),
+                                   FAN_RUN_SLOTS + FAN_SLICE_SLOTS, ms, "pixel*view"),
     }
     rb.close()
     return out
@@ -579,10 +582,10 @@ BWD_SEED = 20261209
 # Algorithmic VALU issue slots of the ray-driven FP and of its transpose,
 # split like the fan BP's into geometry shared by the slices one workgroup
 # carries and work per slice.
-# FP, per ray and image row: the FP64 position step and the inclusion test
-# (2 + 2, FP64 at half rate), the tap index and fraction (2) = 6 per ray-row,
-# shared by the 4 slices of a workgroup; per slice the lerp into the sum, 2.
-# FP^T on the engine, per pixel and view: the channel position (a linear
+# FP, per ray and image row: the 32.32 position step (2), the fraction (2) and
+# the two tap weights (2) = 6 per ray-row, shared by the 4 slices of a wave; per
+# slice the lerp into the sum, 2.
+# FP^T on the view streams, per pixel and view: the channel position (a linear
 # form, 2), its floor and fraction (2), the two tap weights and the edge
 # rule (4) = 8, shared by the 8 slices of a workgroup; per slice 2.
 FP_GEOM_SLOTS, FP_SLICE_SLOTS, FP_SLICES_PER_WG = 6, 2, 4
@@ -950,7 +953,7 @@ def main():
     bp_rate = pv_batch / (ms_bp * 1e-3)
     nb_group = 16
     groups = math.ceil(B / nb_group)
-    slots = pv_slice * FAN_GEOM_SLOTS * groups + pv_batch * FAN_SLICE_SLOTS
+    slots = pv_slice * FAN_RUN_SLOTS * groups + pv_batch * FAN_SLICE_SLOTS
     valu_achieved = slots / (ms_bp * 1e-3)
     hbm_bytes = B * 4 * (na * ns + n * n) + 16 * na + 8 * 2 * n
     hbm_achieved = hbm_bytes / (ms_bp * 1e-3) / 1e9
