@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace ctr {
 
@@ -36,7 +37,7 @@ __device__ inline double cos_weight(const RampParams& P, int is)
     return P.dso * fabs(cos(s / P.dsd)) / P.dsd;
 }
 
-// hf: taps in the accumulation type, hf[ns + m] = h[m]; zero-padded rows in LDS.
+// hf: taps in FP32, hf[ns + m] = h[m]; zero-padded rows in LDS.
 constexpr int kRampNear = 15;  // |m| <= kRampNear: FP64 near field
 
 __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ in,
@@ -107,8 +108,8 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ in,
 // holds, and those in block q - k - 1, which it reads: 16 multiply-adds for 4 reads.
 // Blocks of 8 are stored 10 apart: the lanes' reads meet every bank once.  A wave
 // leaves out the taps that meet only padding.  Each output adds the same products in
-// the same order as in ramp_kernel.  1440 rows of 736: 165 -> 73 us, and the copy of
-// the taps (4 us) is not made.
+// the same order as in ramp_kernel.  1440 rows of 736: 165 -> 40 us (73 with
+// every group's taps clamped), and the copy of the taps (4 us) is not made.
 constexpr int kWideOut = 256;   // outputs of a wave
 constexpr int kWidePitch = 10;  // doubles a block of 8 samples
 // Blocks of padding before the row.  A wave at output i0 takes taps from
@@ -152,15 +153,21 @@ __global__ __launch_bounds__(512) void ramp_f64_kernel(const double* __restrict_
 #pragma unroll
             for (int j = 0; j < 4; ++j) cur[j] = row[-kWidePitch * k + 2 * j];
         };
-        const auto taps = [&](double(&a)[4], int k) {
+        // EDGE: taps past |m| = ns - 1 count as zero (else the four are read at once)
+        const auto taps = [&](auto EDGE, double(&a)[4], int k) {
             double nxt[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) nxt[j] = row[-kWidePitch * (k + 1) + 2 * j];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int m = 8 * k + 1 + 2 * u;
-                const double t = h[ns + min(max(m, 1 - ns), ns - 1)];
-                const double hm = abs(m) < ns ? t : 0.0;
+                double hm;
+                if constexpr (EDGE.value) {
+                    const double t = h[ns + min(max(m, 1 - ns), ns - 1)];
+                    hm = abs(m) < ns ? t : 0.0;
+                } else {
+                    hm = h[ns + m];
+                }
 #pragma unroll
                 for (int j = 0; j < 4; ++j) a[j] = fma(hm, j >= u ? cur[j - u] : nxt[4 + j - u], a[j]);
             }
@@ -171,13 +178,18 @@ __global__ __launch_bounds__(512) void ramp_f64_kernel(const double* __restrict_
         constexpr int kNearLo = -(kRampNear + 1) / 8, kNearHi = kRampNear / 8;
         const int klo = min((i0 - ns) >> 3, kNearLo);
         const int khi = max((i1 - 1) >> 3, kNearHi);
+        // only the first and the last group of a row reach past its taps
+        constexpr std::true_type edge{};
+        constexpr std::false_type inner{};
         load(klo);
+        if (klo < kNearLo) taps(edge, acc, klo);
 #pragma unroll 2
-        for (int k = klo; k < kNearLo; ++k) taps(acc, k);
+        for (int k = klo + 1; k < kNearLo; ++k) taps(inner, acc, k);
 #pragma unroll
-        for (int k = kNearLo; k <= kNearHi; ++k) taps(near, k);
+        for (int k = kNearLo; k <= kNearHi; ++k) taps(edge, near, k);
 #pragma unroll 2
-        for (int k = kNearHi + 1; k <= khi; ++k) taps(acc, k);
+        for (int k = kNearHi + 1; k < khi; ++k) taps(inner, acc, k);
+        if (khi > kNearHi) taps(edge, acc, khi);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int is = 8 * q + p + 2 * j;
