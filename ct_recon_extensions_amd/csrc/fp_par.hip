@@ -285,24 +285,6 @@ int launch_fp(const FpProblem& P, const T* img, const T* imgT, T* proj, const do
     return check_launch("fp_kernel");
 }
 
-// Columns the rays of one fp_stream_kernel chunk can span: 64 channels at up to
-// sqrt(2) ds / pixel per channel, one column per further row, the drift of a ray
-// that is on the image across the other views (at most the image's
-// half-diagonal times sqrt(2) per radian, doubled for the second order), margins.
-bool fp_stream_applies(const ctr_geom& g, int views, int rows, int span_max)
-{
-    const double pmin = std::min(std::fabs(g.dx), std::fabs(g.dy));
-    const double pmax = std::max(std::fabs(g.dx), std::fabs(g.dy));
-    if (!(pmin > 0) || !(g.ds > 0)) return false;
-    const double r = 0.5 * std::hypot(g.nx + 2 * std::fabs(g.offset_x),
-                                      g.ny + 2 * std::fabs(g.offset_y)) * pmax / pmin;
-    const double turn = (views - 1) * std::fabs(g.orbit);
-    const double span = 63 * std::sqrt(2.0) * g.ds / pmin + (rows - 1) * pmax / pmin +
-                        1.5 * r * turn * (1.0 + 2.0 * turn) + 6.0;
-    // steps within 2 columns a row, one plane within a 31-bit buffer range
-    return span <= span_max && pmax <= 1.9 * pmin && 16LL * g.nx * g.ny < (1LL << 31);
-}
-
 // Waves (row segments) per workgroup: 2 where that fills the chip, more for small
 // scans (8 x 512^2, 720 views: 296 us at 2, 303 at 4, 345 at 8; 4 slices 184, 183,
 // 192; one slice 135, 120, 121; 1 x 256^2, 360 views: 68, 54, 54; 8 x 192^2, 200

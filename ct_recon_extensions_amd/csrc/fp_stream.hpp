@@ -26,6 +26,7 @@
 
 #include "bp_engine.hpp"
 #include "ctr_common.hpp"
+#include "fp_span.hpp"
 #include "tile_common.hpp"
 
 namespace ctr {
@@ -124,7 +125,8 @@ __device__ __forceinline__ int wave_min(int x)
 }
 
 // DMA of the chunk's rows k0 .. k0 + kRows - 1, columns cm .. cm + cols - 1, of
-// every plane; columns past the row and rows past the image read as zero.
+// every plane; columns past the row (the last column's right tap is one) and rows
+// past the image read as zero.
 template <int NB, int SPAN>
 __device__ __forceinline__ void fp_stage(const float* src, size_t plane, int nsteps, int rowlen,
                                          int k0, int cm, int cols, int planes, float* buf, int lane)
@@ -134,7 +136,8 @@ __device__ __forceinline__ void fp_stage(const float* src, size_t plane, int nst
     const unsigned int bytes = static_cast<unsigned int>(nsteps) * row_bytes;
     // columns a lane moves: 16 bytes of them, or one where a lane's four would
     // cross the row's end (single slices)
-    const int lane_cols = S::kIl == 4 || cm + ((cols + 3) & ~3) > rowlen ? 1 : 4;
+    const int lane_cols =
+        S::kIl == 4 || (cm + ((cols + 3) & ~3) > rowlen && ((rowlen - cm) & 3)) ? 1 : 4;
     for (int c = 0; c < cols; c += 64 * lane_cols) {
         const int lc = c + lane * lane_cols, col = cm + lc;
         if (lc >= S::kSpan) continue;
@@ -328,11 +331,9 @@ __global__ __launch_bounds__(512) void fp_stream_kernel(const FpStreamLaunch L)
             xmin = fminf(xmin, fmaf(k, sl, lane_value(lo_l, v)));
             xmax = fmaxf(xmax, fmaf(k, sl, lane_value(hi_l, v)));
         }
-        // one column of margin each side (FP32 bounds), the right tap, and the
-        // host's bound on a span (fp_stream_applies)
-        cm_l = min(max(0, static_cast<int>(floorf(fmaxf(xmin, -4.0f))) - 1), rowlen - 1);
-        const int cz = min(rowlen - 1, static_cast<int>(floorf(fminf(xmax, 1e6f))) + 2);
-        cols_l = h0 + lane < nchunks ? min(max(cz - cm_l + 1, 1), S::kSpan) : 0;
+        const FpSpan c = fp_span(xmin, xmax, rowlen, S::kSpan);
+        cm_l = c.first;
+        cols_l = h0 + lane < nchunks ? c.cols : 0;
     };
     spans(0);
     int cm = uniform_i(cm_l);
