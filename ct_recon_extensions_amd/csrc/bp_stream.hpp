@@ -130,7 +130,9 @@ __device__ __forceinline__ StageLane stage_lane(int pitch, int lane)
 // RAW (calls that must not allocate) stages the sinograms as they are, 4 bytes a
 // lane: the same spans, hence the same sums.
 // Off the detector: without EDGE every tap is inside, and what the span holds
-// past the row is not read; with EDGE those channels read as zero (an offset of
+// past the row is not read (past the last row's end a 16-byte load still brings
+// the channels before the end; stream_tile keeps spans before the first row's
+// start out); with EDGE those channels read as zero (an offset of
 // 2^31 is out of range), per lane for 4 slices, else with 4 bytes a lane.
 template <class Geo, int NB, int M, bool EDGE, bool RAW>
 __device__ __forceinline__ void stream_stage(const StreamLaunch<Geo>& L, const StageLane& G,
@@ -412,7 +414,11 @@ __device__ __forceinline__ void stream_tile(const typename Geo::Tables& T,
                 Geo::anchor(P, T, F, va + v, ilo, ilo + kStreamTile - 1, jlo,
                             jlo + kStreamTile - 1);
             anchors[v] = Geo::pack(A);
-            inside = inside && A.inside != 0;
+            // a span that starts at channel -1 of the first view starts before the
+            // buffer, and a 16-byte load there (4 or 2 channels) is out of range as
+            // a whole: channels 0 to 2 with it.  EDGE stages channel by channel.
+            const bool before = S::kIl < 4 && A.is0 < 0 && va + v == 0;
+            inside = inside && A.inside != 0 && !before;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (__ballot(!inside) != 0)

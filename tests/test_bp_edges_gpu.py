@@ -1,0 +1,74 @@
+"""Backprojection where a view's span starts before its sinogram does: one tile, one
+view a wave, the first view's first tap on channel 0.  The span then starts at
+channel -1, four (or two) channels a lane, and the channels from 0 on still count.
+Against the oracle, at the suite's 1e-5 relative L2."""
+import math
+
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.conftest import randn, rel_l2
+
+pytestmark = pytest.mark.gpu
+TOL32 = 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 2, 4])
+@pytest.mark.parametrize("first", [0.3, 0.6, 0.95])
+def test_first_channels_of_the_first_view(n, first):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import ct_recon_extensions_amd as F
+    ns, na, start = 48, 8, 0.1
+    reach = 7.5 * (math.cos(start) + math.sin(start))  # of the tile in view 0, both ways
+    g = dict(nx=16, ny=16, na=na, ns=ns, dx=1.0, dy=1.0, ds=1.0, offset_x=0.0, offset_y=0.0,
+             offset_s=first + reach - (ns - 1) / 2, orbit_start=start, orbit=math.pi / na)
+    og = O.geom(**g)
+    t = O.par_prep(og)
+    proj = randn(1600 + n, (n, na, ns))
+    proj[:, 0, :4] *= 10.0
+    out = F.parallel_backprojection_2d(
+        torch.from_numpy(proj).cuda(), img_shape=[16, 16], img_space=[1.0, 1.0],
+        proj_shape=[na, ns], channel_space=1.0, channel_offset=g["offset_s"], orbit_start=start,
+        orbit=g["orbit"]).cpu().numpy()
+    for b in range(n):
+        assert rel_l2(out[b], O.par_bp(og, proj[b], t)) < TOL32, b
+
+
+@pytest.mark.parametrize("kind", ["ragged", "fan"])
+def test_first_channels_of_the_first_fan_view(kind):
+    """The same for a fan, alone and as a ragged problem's tile."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import numpy as np
+
+    import ct_recon_extensions_amd as F
+    from ct_recon_extensions_amd import ragged
+    from ct_recon_extensions_amd.geometry import FanBackprojection2DAngleParam
+    ns, na, n, dx, ds, dso, dsd = 64, 4, 16, 0.7, 1.3, 595.0, 1085.6
+    # the largest channel distance of a pixel from the centre in the view at angle 0,
+    # found on the pixels themselves
+    x = (np.arange(n) - (n - 1) / 2) * dx
+    s = np.arctan2(x[None, :], dso - x[::-1, None]) * dsd / ds
+    off = 0.6 - s.min() - (ns - 1) / 2
+    angles = 2 * math.pi / na * np.arange(na)
+    og = O.geom(nx=n, ny=n, na=na, ns=ns, dx=dx, dy=dx, ds=ds, offset_x=0.0, offset_y=0.0,
+                offset_s=off, orbit_start=0.0, orbit=2 * math.pi / na, dso=dso, dsd=dsd)
+    proj = randn(1650, (na, ns))
+    proj[0, :4] *= 10.0
+    want = O.fan_bp(og, proj, O.fan_prep(og))
+    if kind == "fan":
+        out = F.fan_backprojection_2d(
+            torch.from_numpy(proj)[None].cuda(), img_shape=[n, n], img_space=[dx, dx],
+            proj_shape=[na, ns], channel_space=ds, channel_offset=off, orbit_start=0.0,
+            orbit=2 * math.pi / na, dso=dso, dsd=dsd)[0]
+    else:
+        p = FanBackprojection2DAngleParam(ns, na, ds, off, n, n, dx, dx, 0.0, 0.0, dso, dsd)
+        plan = ragged.RaggedFanBackprojection2DAngle([p], [angles], autotune=False, tile=0,
+                                                     vchunk=16)
+        plan.projs[0].copy_(torch.from_numpy(proj))
+        out = plan()[0]
+    out = out.cpu().numpy()
+    # (scales differ by a constant)
+    assert rel_l2(out / np.linalg.norm(out), want / np.linalg.norm(want)) < TOL32
