@@ -543,12 +543,19 @@ bool stream_fits(int na, int pitch)
                                stream_vchunk(StreamShape<NB, M>::kViews, NB, pitch)) > 0;
 }
 
-// Whether the stream kernels take a problem: spans of 16 x 16 tiles within
-// kStreamMaxPitch channels, a slice group within a 31-bit buffer range, and
+// Whether the spans of 16 x 16 tiles fit (kStreamMaxPitch channels) and a group of
+// il interleaved sinograms lies within a 31-bit buffer range: row offsets are 32-bit,
+// and the offset of 2^31 of a channel off the detector has to be outside it.
+inline bool stream_reaches(int lmax, long long na, long long ns, int il)
+{
+    return lmax <= kStreamMaxPitch && na * ns * il * 4 < (1LL << 31);
+}
+
+// Whether the stream kernels take a batch: groups of four slices in reach, and
 // views that groups of up to 4 slices always have room for (8 waves of 192).
 inline bool stream_applies(int lmax, long long na, long long ns)
 {
-    return lmax <= kStreamMaxPitch && na * ns * 4 < (1LL << 29) && na <= 8 * 2 * kStreamChain;
+    return stream_reaches(lmax, na, ns, 4) && na <= 8 * 2 * kStreamChain;
 }
 
 // A batch of n sinograms proj, in groups of 16, 8, 4 (2, 1) slices.  A group

@@ -266,7 +266,8 @@ int ctr_ragged_fan_bp_plan(const ctr_ragged_problem* probs, int nprob, int tile,
             D.variant = (exact ? 4 : 0) + cls;
             D.wave_bytes = 0;
             const int order =
-                tile == 0 && !exact && lmax <= kStreamMaxPitch ? fan_run_order(q.g) : 0;
+                tile == 0 && !exact && stream_reaches(lmax, q.g.na, q.g.ns, 1) ? fan_run_order(q.g)
+                                                                                : 0;
             if (order) {
                 D.variant = 7 + order;
                 D.lmax = (lmax + 15) / 16 * 16;  // the staged spans' pitch

@@ -72,3 +72,26 @@ def test_first_channels_of_the_first_fan_view(kind):
     out = out.cpu().numpy()
     # (scales differ by a constant)
     assert rel_l2(out / np.linalg.norm(out), want / np.linalg.norm(want)) < TOL32
+
+
+def test_ragged_sinogram_of_more_than_4_gib():
+    """The stream tile reaches a sinogram through 31 bits of bytes; a longer one is the
+    engine tile's.  2^28 channels, of which the image uses the middle 120."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import numpy as np
+
+    from ct_recon_extensions_amd import ragged
+    from ct_recon_extensions_amd.geometry import FanBackprojection2DAngleParam
+    na, n, few, ns = 5, 40, 120, 1 << 28
+    angles = 2 * math.pi / na * np.arange(na)
+    og = O.geom(nx=n, ny=n, na=na, ns=few, dx=0.7, dy=0.7, ds=1.3, offset_x=0.0, offset_y=0.0,
+                offset_s=0.0, orbit_start=0.0, orbit=2 * math.pi / na, dso=595.0, dsd=1085.6)
+    proj = randn(1660, (na, few))
+    want = O.fan_bp(og, proj, O.fan_prep(og))
+    p = FanBackprojection2DAngleParam(ns, na, 1.3, 0.0, n, n, 0.7, 0.7, 0.0, 0.0, 595.0, 1085.6)
+    plan = ragged.RaggedFanBackprojection2DAngle([p], [angles], autotune=False, tile=0, vchunk=16)
+    a = (ns - few) // 2
+    plan.projs[0][:, a:a + few] = torch.from_numpy(proj).cuda()
+    out = plan()[0].cpu().numpy()
+    assert rel_l2(out / np.linalg.norm(out), want / np.linalg.norm(want)) < TOL32
