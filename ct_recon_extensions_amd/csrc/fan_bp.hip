@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restric
     const double fi = x - xc, fj = yc - y;
     const size_t sino = static_cast<size_t>(P.na) * P.ns;
     const double* src = proj + static_cast<size_t>(b0) * sino;
-    const double last = P.ns - 1, half = 0.5 * last;
+    const double last = P.ns - 1;
     double sum[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) sum[b] = 0.0;
@@ -149,30 +149,33 @@ __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restric
                 q = fma(t, q, -1.0);
                 q = fma(t, q, 1.0);
                 double s = fma(fma(u * t, a, u), P.kd, A.sc);
-                // at the detector's ends a whole tap hangs on the last bit of s:
-                // there it is the reference's expression
-                const double c = fabs(s - half) - half;
-                bool on = c < 0;
-                if (fabs(c) < 1e-9) {
+                // at a whole channel the taps hang on the last bit of s (the ends of
+                // the detector, and one tap or two): there it is the reference's
+                // expression
+                bool on = s > 0 && s < last;
+                double fl = floor(s);
+                if (fabs(s - fl - 0.5) > 0.5 - 1e-9) {
                     const double sb = T.sincos[2 * (va + vv)], cb = T.sincos[2 * (va + vv) + 1];
                     s = atan2(x * cb + y * sb, P.dso + x * sb - y * cb) * P.dsd / P.ds + P.cents;
                     on = s >= 0 && s <= last;
+                    fl = floor(s);
                 }
                 on = on && v + k < nva;
-                const double fl = floor(s), w = on ? rd * rd * q : 0.0;
+                const double w = on ? rd * rd * q : 0.0;
                 w1[k] = on ? w * (s - fl) : 0.0;
                 w0[k] = w - w1[k];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) p0[k][b] = p1[k][b] = 0.0;
                 if (on) {
-                    const int i = static_cast<int>(fl);
+                    // floor(s) and ceil(s)
+                    const int i = static_cast<int>(fl), j = i + (fl < s ? 1 : 0);
                     const double* row = src + static_cast<size_t>(va + vv) * P.ns;
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
                         // a slice past the batch re-reads the last one
                         const size_t o = static_cast<size_t>(min(b, nb - 1)) * sino;
                         p0[k][b] = row[o + i];
-                        p1[k][b] = row[o + min(i + 1, P.ns - 1)];
+                        p1[k][b] = row[o + j];
                     }
                 }
             }

@@ -95,3 +95,33 @@ def test_ragged_sinogram_of_more_than_4_gib():
     plan.projs[0][:, a:a + few] = torch.from_numpy(proj).cuda()
     out = plan()[0].cpu().numpy()
     assert rel_l2(out / np.linalg.norm(out), want / np.linalg.norm(want)) < TOL32
+
+
+@pytest.mark.parametrize("n", [1, 2, 4])
+def test_float64_integer_positions_read_one_channel(n):
+    """A pixel whose position is a whole channel (the central rays of an odd detector)
+    reads that channel only, as the reference's floor(s) and ceil(s) do: inf and nan
+    next to it stay out of its sum."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import numpy as np
+
+    import ct_recon_extensions_amd as F
+    ns, na, side = 45, 12, 33
+    g = dict(nx=side, ny=side, na=na, ns=ns, dx=0.7, dy=0.7, ds=1.3, offset_x=0.0, offset_y=0.0,
+             offset_s=0.0, orbit_start=0.0, orbit=2 * math.pi / na, dso=595.0, dsd=1085.6)
+    og = O.geom(**g)
+    t = O.fan_prep(og)
+    proj = np.random.default_rng(1670).standard_normal((n, na, ns))
+    c = (ns - 1) // 2
+    proj[0, 0, c + 1], proj[0, 3, c + 1], proj[0, 5, c - 1] = np.inf, np.nan, -np.inf
+    out = F.fan_backprojection_2d(
+        torch.from_numpy(proj).cuda(), img_shape=[side, side], img_space=[0.7, 0.7],
+        proj_shape=[na, ns], channel_space=1.3, channel_offset=0.0, orbit_start=0.0,
+        orbit=g["orbit"], dso=595.0, dsd=1085.6).cpu().numpy()
+    assert np.isfinite(out[0, 16, 16])
+    for b in range(n):
+        want = O.fan_bp(og, proj[b], t)
+        np.testing.assert_array_equal(np.isfinite(out[b]), np.isfinite(want))
+        ok = np.isfinite(want)
+        assert rel_l2(out[b][ok], want[ok]) < 1e-12, b
