@@ -63,17 +63,20 @@ __global__ void plain_fan_bp_kernel(const T* __restrict__ proj, T* __restrict__ 
 //     u = num / den (a reciprocal from v_rcp_f64 and two Newton steps),
 //     s = s_c + k atan(u),  w = (dsd / (Lc (1 + e)))^2 / (1 + u^2),
 // with the series of atan and 1 / (1 + u^2) to u^15 and u^16: below 1e-17 for |u|
-// <= 0.1, which the host checks.  The offsets are small, so s
-// keeps the rounding of s_c; sums run over the views in their order.
-// 2 x 512^2, 720 views, 736 channels: 1.58 -> 0.49 ms, of which the vector units
-// issue 0.31 and the test at the detector's ends takes 0.03; four views at a time and
-// both taps in one 16-byte load were 0.02 ms slower, a bound of 96 registers (spills)
-// 0.2 ms.
+// <= 0.1, which the host checks.  s_c is kept as a whole channel and a fraction, so
+// a position carries the rounding of the anchor's angle alone: 1.9e-14 channel rms
+// against the reference expression's 2.8e-14 (512^2 over 736 channels; with s_c
+// rounded to one double 3.4e-14).  Sums run over the views in their order.
+// 2 x 512^2, 720 views, 736 channels, in a kernel trace: 1.58 -> 0.51 ms, of which
+// the vector units issue 0.31 (one view at a time 0.54, four 0.51; both taps in one
+// 16-byte load was 0.02 slower, a bound of 96 registers, which spills, 0.2).
 struct FanAnchor64 {
-    double ui, uj, bi, bj, b0, sc;
+    double ui, uj, bi, bj, b0, frac;  // the anchor's position is whole + frac channels
+    int whole;
 };
-constexpr int kFan64Views = 128;  // anchors per round (6 KB of LDS)
+constexpr int kFan64Views = 128;  // anchors per round (7 KB of LDS)
 constexpr int kFan64Unroll = 2;
+static_assert(kFan64Views % kFan64Unroll == 0, "views in flight within a round");
 
 template <int NB>
 __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restrict__ proj,
@@ -97,7 +100,6 @@ __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restric
     const double fi = x - xc, fj = yc - y;
     const size_t sino = static_cast<size_t>(P.na) * P.ns;
     const double* src = proj + static_cast<size_t>(b0) * sino;
-    const double last = P.ns - 1;
     double sum[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) sum[b] = 0.0;
@@ -115,17 +117,22 @@ __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restric
             A.bi = (sb * d + cb * r) * inv * iq;
             A.bj = (cb * d - sb * r) * inv * iq;
             A.b0 = iq;
-            A.sc = atan2(r, d) * P.dsd / P.ds + P.cents;
+            const double sc = atan2(r, d) * P.dsd / P.ds, wh = floor(sc + P.cents);
+            A.frac = sc - (wh - P.cents);
+            A.whole = static_cast<int>(wh);
             anchors[tid] = A;
+        } else if (tid < kFan64Views) {
+            // past the last view: off the detector
+            anchors[tid] = FanAnchor64{0.0, 0.0, 0.0, 0.0, 1.0, 0.5, -(1 << 30)};
         }
         __syncthreads();
         // kFan64Unroll views at a time: their chains of dependent FP64 operations
-        // and their loads overlap (one at a time: 0.47 ms)
+        // and their loads overlap
         for (int v = 0; v < nva; v += kFan64Unroll) {
             double p0[kFan64Unroll][NB], p1[kFan64Unroll][NB], w0[kFan64Unroll], w1[kFan64Unroll];
 #pragma unroll
             for (int k = 0; k < kFan64Unroll; ++k) {
-                const int vv = min(v + k, nva - 1);
+                const int vv = v + k;
                 const FanAnchor64 A = anchors[vv];
                 const double num = fma(A.ui, fi, A.uj * fj);
                 const double den = fma(A.bi, fi, fma(A.bj, fj, A.b0));
@@ -148,27 +155,29 @@ __global__ __launch_bounds__(256) void fan_bp_f64_kernel(const double* __restric
                 q = fma(t, q, 1.0);
                 q = fma(t, q, -1.0);
                 q = fma(t, q, 1.0);
-                double s = fma(fma(u * t, a, u), P.kd, A.sc);
+                const double s = fma(fma(u * t, a, u), P.kd, A.frac);
+                double fl = floor(s), fr = s - fl;
+                int i = A.whole + static_cast<int>(fl);
+                bool on = static_cast<unsigned int>(i) < static_cast<unsigned int>(P.ns - 1);
                 // at a whole channel the taps hang on the last bit of s (the ends of
                 // the detector, and one tap or two): there it is the reference's
                 // expression
-                bool on = s > 0 && s < last;
-                double fl = floor(s);
-                if (fabs(s - fl - 0.5) > 0.5 - 1e-9) {
+                if (fabs(fr - 0.5) > 0.5 - 1e-9) {
                     const double sb = T.sincos[2 * (va + vv)], cb = T.sincos[2 * (va + vv) + 1];
-                    s = atan2(x * cb + y * sb, P.dso + x * sb - y * cb) * P.dsd / P.ds + P.cents;
-                    on = s >= 0 && s <= last;
-                    fl = floor(s);
+                    const double se =
+                        atan2(x * cb + y * sb, P.dso + x * sb - y * cb) * P.dsd / P.ds + P.cents;
+                    on = se >= 0 && se <= P.ns - 1;
+                    fl = floor(se);
+                    fr = se - fl;
+                    i = static_cast<int>(fl);
                 }
-                on = on && v + k < nva;
                 const double w = on ? rd * rd * q : 0.0;
-                w1[k] = on ? w * (s - fl) : 0.0;
+                w1[k] = w * fr;
                 w0[k] = w - w1[k];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) p0[k][b] = p1[k][b] = 0.0;
                 if (on) {
-                    // floor(s) and ceil(s)
-                    const int i = static_cast<int>(fl), j = i + (fl < s ? 1 : 0);
+                    const int j = i + (fr > 0 ? 1 : 0);  // ceil(s)
                     const double* row = src + static_cast<size_t>(va + vv) * P.ns;
 #pragma unroll
                     for (int b = 0; b < NB; ++b) {
