@@ -21,12 +21,16 @@
 //  * a wave evaluates the FP64 anchors of all its views first (64 at a time,
 //    one a lane) and keeps them in LDS, while no sum is live in registers.
 // Sums: one FP32 chain of at most kStreamChain views a lane, the halves of a
-// wave added in FP32, the waves in FP64.
+// wave added in FP32, the waves in FP64.  The split depends on the batch: runs are
+// of 4 pixels in groups of 16 slices and of 8 in smaller ones (the sums of 16 x 8
+// pixels do not fit the registers), and the wave count follows the number of
+// workgroups.  So a slice's last bits are those of its batch size.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "bp_engine.hpp"
 #include "ctr_common.hpp"
@@ -127,8 +131,8 @@ __device__ __forceinline__ StageLane stage_lane(int pitch, int lane)
 // itself), so a lane moves 16 bytes: 4, 2 or 1 channels of 1, 2 or 4 slices.  With
 // 4 bytes a lane, the slices apart, the DMAs of 4-slice groups cost as much as
 // the sums (the 4-slice BP of 512^2, 720 views: 227 us against 150).
-// RAW (calls that must not allocate) stages the sinograms as they are, 4 bytes a
-// lane: the same spans, hence the same sums.
+// RAW (calls that must not or cannot allocate) stages the sinograms as they are, 4
+// bytes a lane: the same spans, hence the same sums.
 // Off the detector: without EDGE every tap is inside, and what the span holds
 // past the row is not read (past the last row's end a 16-byte load still brings
 // the channels before the end; stream_tile keeps spans before the first row's
@@ -573,7 +577,7 @@ int launch_stream_part(StreamLaunch<Geo> L, const typename Geo::Tables& T, const
     float* ws = nullptr;
     if (n > 1 && !RAW) {
         const size_t slices = n == 2 ? 2 : div_up(n, 4) * 4;
-        const int e = ws_part(reinterpret_cast<void**>(&ws), slices * sino * sizeof(float), n, st);
+        const int e = ws_part(reinterpret_cast<void**>(&ws), slices * sino * sizeof(float), st);
         if (e) return e;
         const dim3 grid(div_up(sino, 256), n == 2 ? 1 : div_up(n, 4));
         if (n == 2)
@@ -613,14 +617,17 @@ template <class Geo, bool RAW = false>
 int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, const float* proj,
                         int n, int lmax, hipStream_t st)
 {
-    if (RAW) return launch_stream_part<Geo, true>(L, T, proj, n, lmax, st);
+    if constexpr (RAW) return launch_stream_part<Geo, true>(L, T, proj, n, lmax, st);
     const size_t sino = static_cast<size_t>(L.P.na) * L.P.ns;
     const size_t image = static_cast<size_t>(L.P.nx) * L.P.ny;
     float* const img = L.img;
-    return in_parts(n, sino * sizeof(float), [&](int b, int count) {
+    const auto part = [&](auto raw, int b, int count) {
         L.img = img + b * image;
-        return launch_stream_part<Geo>(L, T, proj + b * sino, count, lmax, st);
-    });
+        return launch_stream_part<Geo, decltype(raw)::value>(L, T, proj + b * sino, count, lmax, st);
+    };
+    return in_parts(
+        n, sino * sizeof(float), [&](int b, int count) { return part(std::false_type{}, b, count); },
+        [&](int b, int count) { return part(std::true_type{}, b, count); });
 }
 
 }  // namespace ctr

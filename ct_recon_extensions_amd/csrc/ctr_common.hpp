@@ -58,13 +58,14 @@ hipError_t ws_free(void* p, hipStream_t st);
 
 // A batch in parts whose scratch (bytes a slice) stays within 1 GiB, at least 16
 // slices each: call(first, count).  A part whose scratch the device has no room for
-// (ws_part: kNoScratch) is called slice by slice, which needs next to none.
+// (ws_part: kNoScratch) is small(first, count)'s, which gets by with less and gives the
+// same bits: what is free on the device does not show in a result.
 constexpr int kNoScratch = -1;
 
-inline int ws_part(void** p, size_t bytes, int count, hipStream_t st)
+inline int ws_part(void** p, size_t bytes, hipStream_t st)
 {
     const hipError_t e = ws_alloc(p, bytes, st);
-    if (e == hipErrorOutOfMemory && count > 1) {
+    if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
         return kNoScratch;
     }
@@ -72,8 +73,8 @@ inline int ws_part(void** p, size_t bytes, int count, hipStream_t st)
     return 0;
 }
 
-template <typename F>
-int in_parts(int n, size_t bytes, F&& call)
+template <typename F, typename G>
+int in_parts(int n, size_t bytes, F&& call, G&& small)
 {
     const size_t fit = (size_t{1} << 30) / bytes / 16 * 16;
     const int part = static_cast<int>(fit < 16 ? 16 : fit < static_cast<size_t>(n) ? fit : n);
@@ -81,10 +82,19 @@ int in_parts(int n, size_t bytes, F&& call)
     for (int b = 0; b < n && rc == 0; b += part) {
         const int count = n - b < part ? n - b : part;
         rc = call(b, count);
-        if (rc != kNoScratch) continue;
-        rc = 0;
-        for (int i = 0; i < count && rc == 0; ++i) rc = call(b + i, 1);
+        if (rc == kNoScratch) rc = small(b, count);
     }
+    if (rc != kNoScratch) return rc;
+    set_error("out of device memory");
+    return CTR_ERR_HIP;
+}
+
+// small() of operators that take the slices of a part one at a time.
+template <typename F>
+int one_by_one(int first, int count, F&& call)
+{
+    int rc = 0;
+    for (int i = 0; i < count && rc == 0; ++i) rc = call(first + i);
     return rc;
 }
 

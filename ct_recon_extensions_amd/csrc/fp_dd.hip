@@ -538,7 +538,7 @@ int fp_dd_f32_part(const ctr_geom& g, const float* img, float* proj, int nbatch,
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     float* ws = nullptr;
     const int e = ws_part(reinterpret_cast<void**>(&ws),
-                          (8 * np + (single ? 2 : 0)) * slice * sizeof(float), nbatch, st);
+                          (8 * np + (single ? 2 : 0)) * slice * sizeof(float), st);
     if (e) return e;
     float *rows = ws, *cols = ws + 4 * np * slice, *one = ws + 8 * np * slice;
     const dim3 tiles(div_up(g.nx, 32), div_up(g.ny, 32)), block(32, 8);
@@ -579,7 +579,7 @@ int fp_dd_grad_f32_part(const ctr_geom& g, const float* proj, float* img, int nb
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     float* ws = nullptr;
     if (np) {
-        const int e = ws_part(reinterpret_cast<void**>(&ws), 4 * np * sino * sizeof(float), nbatch, st);
+        const int e = ws_part(reinterpret_cast<void**>(&ws), 4 * np * sino * sizeof(float), st);
         if (e) return e;
         hipLaunchKernelGGL(interleave_kernel<4>, dim3(div_up(sino, 256), np), dim3(256), 0, st,
                            proj, ws, static_cast<unsigned int>(sino), nbatch);
@@ -609,8 +609,11 @@ int fp_dd_f32(const ctr_geom& g, const float* img, float* proj, int nbatch, cons
               const double* bo, const int* usex, hipStream_t st)
 {
     const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
-    return in_parts(nbatch, 2 * slice * sizeof(float), [&](int b, int count) {
+    const auto part = [&](int b, int count) {
         return fp_dd_f32_part(g, img + b * slice, proj + b * sino, count, sc, bo, usex, st);
+    };
+    return in_parts(nbatch, 2 * slice * sizeof(float), part, [&](int b, int count) {
+        return one_by_one(b, count, [&](int i) { return part(i, 1); });
     });
 }
 
@@ -618,9 +621,12 @@ int fp_dd_grad_f32(const ctr_geom& g, const float* proj, float* img, int nbatch,
                    const double* pos, const int* usex, int stride, hipStream_t st)
 {
     const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
-    return in_parts(nbatch, sino * sizeof(float), [&](int b, int count) {
+    const auto part = [&](int b, int count) {
         return fp_dd_grad_f32_part(g, proj + b * sino, img + b * slice, count, w, pos, usex, stride,
                                    st);
+    };
+    return in_parts(nbatch, sino * sizeof(float), part, [&](int b, int count) {
+        return one_by_one(b, count, [&](int i) { return part(i, 1); });
     });
 }
 

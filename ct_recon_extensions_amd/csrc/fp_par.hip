@@ -288,33 +288,39 @@ int launch_fp(const FpProblem& P, const T* img, const T* imgT, T* proj, const do
 // Waves (row segments) per workgroup: 2 where that fills the chip, more for small
 // scans (8 x 512^2, 720 views: 296 us at 2, 303 at 4, 345 at 8; 4 slices 184, 183,
 // 192; one slice 135, 120, 121; 1 x 256^2, 360 views: 68, 54, 54; 8 x 192^2, 200
-// views: 61, 55, 61).
+// views: 61, 55, 61).  groups: slice groups of the launch.
+int fp_stream_waves(const ctr_geom& g, int shape, int groups)
+{
+    const int vgroups = div_up(g.na, shape < 2 ? 4 : 1);
+    return static_cast<long long>(div_up(g.ns, 64)) * vgroups * groups >= 4096 ? 2 : 4;
+}
+
+// Segments are whole fours of rows for any NB: a slice alone has the sums that it
+// has in a group of four with as many waves.
 template <int NB, int V, int SPAN>
-int launch_fp_stream_s(FpStreamLaunch L, int n, hipStream_t st)
+int launch_fp_stream_s(FpStreamLaunch L, int n, int waves, hipStream_t st)
 {
     using S = FpShape<NB, SPAN>;
+    static_assert(4 % S::kRows == 0, "segments of whole chunks");
     L.nb = n;
     L.cgroups = div_up(L.P.ns, 64);
     const int groups = div_up(n, NB), vgroups = div_up(L.P.na, V);
-    const int steps = std::max(L.P.nx, L.P.ny);
-    const long long blocks = static_cast<long long>(L.cgroups) * vgroups * groups;
-    const int w = blocks >= 4096 ? 2 : 4;
-    L.chunks = div_up(div_up(steps, S::kRows), w);
-    const size_t lds = static_cast<size_t>(w) * S::kLds;
+    L.chunks = div_up(div_up(std::max(L.P.nx, L.P.ny), 4), waves) * (4 / S::kRows);
+    const size_t lds = static_cast<size_t>(waves) * S::kLds;
     hipLaunchKernelGGL((fp_stream_kernel<NB, V, SPAN>), dim3(L.cgroups * vgroups, groups, 2),
-                       dim3(64 * w), lds, st, L);
+                       dim3(64 * waves), lds, st, L);
     return check_launch("fp_stream_kernel");
 }
 
 // shape: 0 4 views and 128 columns, 1 4 and 256, 2 1 and 128, 3 1 and 256.
 template <int NB>
-int launch_fp_stream(int shape, const FpStreamLaunch& L, int n, hipStream_t st)
+int launch_fp_stream(int shape, const FpStreamLaunch& L, int n, int waves, hipStream_t st)
 {
     switch (shape) {
-        case 0: return launch_fp_stream_s<NB, 4, 128>(L, n, st);
-        case 1: return launch_fp_stream_s<NB, 4, 256>(L, n, st);
-        case 2: return launch_fp_stream_s<NB, 1, 128>(L, n, st);
-        default: return launch_fp_stream_s<NB, 1, 256>(L, n, st);
+        case 0: return launch_fp_stream_s<NB, 4, 128>(L, n, waves, st);
+        case 1: return launch_fp_stream_s<NB, 4, 256>(L, n, waves, st);
+        case 2: return launch_fp_stream_s<NB, 1, 128>(L, n, waves, st);
+        default: return launch_fp_stream_s<NB, 1, 256>(L, n, waves, st);
     }
 }
 
@@ -328,8 +334,10 @@ int fp_stream_shape(const ctr_geom& g)
     return -1;
 }
 
-int fp_stream_part(const ctr_geom& g, int shape, const float* img, float* proj, int nbatch, const double* sc,
-              const double* bo, const int* usex, hipStream_t st)
+// waves: of the groups of four; waves1: of a last slice alone.
+int fp_stream_part(const ctr_geom& g, int shape, int waves, int waves1, const float* img,
+                   float* proj, int nbatch, const double* sc, const double* bo, const int* usex,
+                   hipStream_t st)
 {
     FpStreamLaunch L{};
     L.P = FpProblem{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
@@ -343,7 +351,7 @@ int fp_stream_part(const ctr_geom& g, int shape, const float* img, float* proj, 
     const bool single = nbatch % 4 == 1;  // the last slice alone
     float* ws = nullptr;
     const int e = ws_part(reinterpret_cast<void**>(&ws),
-                          (8 * np + (single ? 1 : 0)) * slice * sizeof(float), nbatch, st);
+                          (8 * np + (single ? 1 : 0)) * slice * sizeof(float), st);
     if (e) return e;
     float *rows = ws, *cols = ws + 4 * np * slice, *one = ws + 8 * np * slice;
     const dim3 tiles(div_up(g.nx, 32), div_up(g.ny, 32), std::max(np, 1));
@@ -362,11 +370,11 @@ int fp_stream_part(const ctr_geom& g, int shape, const float* img, float* proj, 
         L.cols = cols;
         if (left >= 2) {
             take = left % 4 == 1 ? left - 1 : left;
-            rc = launch_fp_stream<4>(shape, L, take, st);
+            rc = launch_fp_stream<4>(shape, L, take, waves, st);
         } else {
             L.rows = img;                   // indexed by slice
             L.cols = one - b0 * slice;
-            rc = launch_fp_stream<1>(shape, L, 1, st);
+            rc = launch_fp_stream<1>(shape, L, 1, waves1, st);
         }
         b0 += take;
     }
@@ -378,9 +386,19 @@ int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int n
               const double* sc, const double* bo, const int* usex, hipStream_t st)
 {
     const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
-    return in_parts(nbatch, 2 * slice * sizeof(float), [&](int b, int count) {
-        return fp_stream_part(g, shape, img + b * slice, proj + b * sino, count, sc, bo, usex, st);
-    });
+    // of the whole call, whatever its parts are
+    const int four = nbatch % 4 == 1 ? nbatch - 1 : nbatch;  // slices in groups of four
+    const int waves = fp_stream_waves(g, shape, div_up(four, 4));
+    const int waves1 = fp_stream_waves(g, shape, 1);
+    const auto part = [&](int b, int count, int w1) {
+        return fp_stream_part(g, shape, waves, w1, img + b * slice, proj + b * sino, count, sc, bo,
+                              usex, st);
+    };
+    return in_parts(
+        nbatch, 2 * slice * sizeof(float), [&](int b, int count) { return part(b, count, waves1); },
+        [&](int b, int count) {
+            return one_by_one(b, count, [&](int i) { return part(i, 1, i < four ? waves : waves1); });
+        });
 }
 
 template <typename T>

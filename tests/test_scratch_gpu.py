@@ -1,0 +1,83 @@
+"""A call whose scratch the device has no room for gives the bits that it gives with
+room.  The room is taken away by a hipMallocAsync of our own, which a child process puts
+before the runtime's and which refuses blocks above a limit."""
+import os
+import subprocess
+import sys
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
+
+SHIM = r"""
+#include <cstddef>
+#include <dlfcn.h>
+static size_t g_limit = ~size_t{0};
+static int g_refused = 0;
+extern "C" {
+void limit(size_t n) { g_limit = n; }
+int refused() { return g_refused; }
+int hipMallocAsync(void** p, size_t n, void* stream)
+{
+    using F = int (*)(void**, size_t, void*);
+    static F real = (F)dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMallocAsync");
+    if (n <= g_limit) return real(p, n, stream);
+    ++g_refused;
+    return 2;  // hipErrorOutOfMemory
+}
+}
+"""
+
+CHILD = r"""
+import ctypes as C, math, sys
+shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+shim.limit.argtypes = [C.c_size_t]
+sys.path.insert(0, sys.argv[2])
+import torch
+import ct_recon_extensions_amd as F
+from ct_recon_extensions_amd import _lib
+_lib.load()
+torch.manual_seed(3)
+na, ns, side = 90, 96, 70
+kw = dict(img_shape=[side, side], img_space=[0.7, 0.7], proj_shape=[na, ns], channel_space=1.3,
+          orbit=math.pi / na)
+fan = dict(kw, orbit=2 * math.pi / na, dso=595.0, dsd=1085.6)
+ops = {
+    "fan": lambda n: F.fan_backprojection_2d(sino[:n], **fan),
+    "par": lambda n: F.parallel_backprojection_2d(sino[:n], **kw),
+    "fp": lambda n: F.parallel_projection_2d(img[:n], **kw),
+    "dd": lambda n: F.parallel_projection_2d(img[:n], method="disdriven", **kw),
+    "ddg": lambda n: F.parallel_projection_2d_grad(sino[:n], method="disdriven", **kw),
+}
+sino = torch.randn((35, na, ns), device="cuda")
+img = torch.randn((35, side, side), device="cuda")
+for name, op in ops.items():
+    for n in (2, 3, 5, 8, 9, 11, 17, 18, 35):
+        shim.limit(1 << 40)
+        want = op(n)
+        torch.cuda.synchronize()
+        _lib.call("ctr_release_workspace")
+        shim.limit(65536)  # one slice's scratch, not two's
+        before = shim.refused()
+        got = op(n)
+        torch.cuda.synchronize()
+        assert shim.refused() > before, (name, n)
+        assert torch.equal(got, want), (name, n)
+        _lib.call("ctr_release_workspace")
+print("same bits")
+"""
+
+
+def test_results_do_not_depend_on_free_memory(tmp_path):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    (tmp_path / "shim.cpp").write_text(SHIM)
+    (tmp_path / "child.py").write_text(CHILD)
+    so = str(tmp_path / "shim.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(tmp_path / "shim.cpp"), "-o", so, "-ldl"],
+                   check=True)
+    r = subprocess.run([sys.executable, str(tmp_path / "child.py"), so, ROOT], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and "same bits" in r.stdout, r.stdout + r.stderr[-2000:]
