@@ -9,7 +9,8 @@
 // for the event is then satisfied by the stream's order), a call on another
 // stream only a block whose event has passed.  At most kKeep bytes and
 // kBlocks blocks are kept free, the oldest go first, and ctr_release_workspace
-// gives them all back.  Any number of threads and streams: a block belongs to
+// gives them all back to the device (an allocator beside this one, PyTorch's for
+// one, cannot ask for them).  Any number of threads and streams: a block belongs to
 // one call from ws_alloc to ws_free.
 #include <cstdint>
 #include <deque>
@@ -23,7 +24,7 @@ namespace ctr {
 namespace {
 
 // 1 GiB: the scratch of the largest sinogram batch of the benchmark (32 x 1440
-// x 1472) four times over
+// x 1472: 259 MiB, a block of 320) three times over
 constexpr size_t kKeep = size_t{1} << 30, kBlocks = 64;
 
 struct Block {
@@ -170,6 +171,11 @@ extern "C" int ctr_release_workspace(void)
             (void)hipEventDestroy(b.done);
             CTR_HIP(hipFree(b.p));
         }
+        // the pool behind hipMallocAsync would hold on to them until the next
+        // synchronisation
+        hipMemPool_t pool = nullptr;
+        CTR_HIP(hipDeviceGetDefaultMemPool(&pool, dev));
+        CTR_HIP(hipMemPoolTrimTo(pool, 0));
         return CTR_OK;
     } catch (const std::exception& e) {
         set_error(std::string("ctr_release_workspace: ") + e.what());

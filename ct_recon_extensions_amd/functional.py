@@ -32,11 +32,20 @@ __all__ = [
     "parallel_backprojection_2d_grad", "parallel_projection_2d", "parallel_projection_2d_grad",
     "fan_backprojection_2d", "fan_backprojection_2d_grad", "fan_backprojection_2d_angle",
     "fan_backprojection_2d_angle_grad", "fan_weighting", "fan_weighting_grad",
-    "helical_interpolation",
+    "helical_interpolation", "release_workspace",
 ]
 
 _FILTER_TYPES = {"par": 0, "fan": 1, "flat": 2}
 _WEIGHT_TYPES = {"fan": 1, "flat": 2}
+
+
+def release_workspace(device=None) -> None:
+    """Give the scratch memory that the operators keep between calls (up to 1 GiB a
+    device) back to ``device`` (default: the current one), once its last uses are done.
+    PyTorch's allocator cannot ask for it: call this, beside
+    ``torch.cuda.empty_cache()``, before something that needs all of the memory."""
+    with torch.cuda.device(device):
+        _lib.call("ctr_release_workspace")
 
 
 # ---------------------------------------------------------------- helpers

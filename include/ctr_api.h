@@ -62,7 +62,7 @@ const char* ctr_last_error(void);
 /* Library version as 10000*major + 100*minor + patch. */
 int ctr_version(void);
 /* Operators keep up to 1 GiB of scratch memory per device between calls; this
- * waits for its last uses and gives the current device's back. */
+ * waits for its last uses and gives the current device's back to the device. */
 int ctr_release_workspace(void);
 /* Device properties the kernels are tuned on (for reports). */
 int ctr_device_info(int* cu_count, int* clock_khz, int* lds_bytes_per_cu, char* arch,

@@ -81,3 +81,25 @@ def test_results_do_not_depend_on_free_memory(tmp_path):
     r = subprocess.run([sys.executable, str(tmp_path / "child.py"), so, ROOT], capture_output=True,
                        text=True, timeout=100)
     assert r.returncode == 0 and "same bits" in r.stdout, r.stdout + r.stderr[-2000:]
+
+
+def test_release_workspace_gives_memory_back_to_the_device():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import math
+
+    import ct_recon_extensions_amd as F
+    kw = dict(img_shape=[16, 16], img_space=[0.7, 0.7], proj_shape=[1440, 5888], channel_space=1.3,
+              orbit=2 * math.pi / 1440, dso=595.0, dsd=1085.6)
+    x = torch.zeros((8, 1440, 5888), device="cuda")
+    scratch = x.numel() * 4
+    F.fan_backprojection_2d(x[:1], **kw)  # tables
+    F.release_workspace()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    y = F.fan_backprojection_2d(x, **kw)
+    torch.cuda.synchronize()
+    kept = torch.cuda.mem_get_info()[0]
+    assert before - kept >= scratch
+    F.release_workspace(y.device)
+    assert torch.cuda.mem_get_info()[0] - kept >= scratch

@@ -58,6 +58,8 @@ hipError_t hipFreeAsync(void* p, hipStream_t)
     g_live.erase(it);
     return hipSuccess;
 }
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
 hipError_t hipFree(void* p) { return hipFreeAsync(p, nullptr); }
 }
 
