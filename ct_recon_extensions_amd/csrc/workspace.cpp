@@ -61,6 +61,15 @@ bool capturing(hipStream_t st)
     return status != hipStreamCaptureStatusNone;
 }
 
+// Another thread may be capturing a graph, which (in the global mode, PyTorch's
+// default) calls like hipEventQuery and hipMallocAsync from any thread would
+// invalidate; none of those made here touches a captured stream.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 }  // namespace
 
 hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
@@ -71,6 +80,7 @@ hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     const size_t want = block_size(bytes);
+    const RelaxedCapture relaxed;
     try {
         std::lock_guard<std::mutex> lock(g_mu);
         Device& D = g_devices[dev];
@@ -126,6 +136,7 @@ hipError_t ws_free(void* p, hipStream_t st)
         std::lock_guard<std::mutex> lock(g_mu);
         const auto it = g_used.find(p);
         if (it == g_used.end()) return hipFreeAsync(p, st);  // a captured allocation
+        const RelaxedCapture relaxed;
         Block b = it->second;
         g_used.erase(it);
         b.st = st;
@@ -162,6 +173,7 @@ extern "C" int ctr_release_workspace(void)
         std::lock_guard<std::mutex> lock(g_mu);
         int dev = 0;
         CTR_HIP(hipGetDevice(&dev));
+        const RelaxedCapture relaxed;
         Device& D = g_devices[dev];
         while (!D.free.empty()) {
             const Block b = D.free.back();

@@ -103,3 +103,70 @@ def test_release_workspace_gives_memory_back_to_the_device():
     assert before - kept >= scratch
     F.release_workspace(y.device)
     assert torch.cuda.mem_get_info()[0] - kept >= scratch
+
+
+def test_calls_beside_another_threads_capture():
+    """Operators that take scratch (kept blocks of other streams, new ones) while
+    another thread captures a graph neither fail nor invalidate the capture."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import ctypes as C
+    import math
+    import threading
+
+    import ct_recon_extensions_amd as F
+    from ct_recon_extensions_amd import _lib
+    from ct_recon_extensions_amd.geometry import FanBackprojection2DParam, device_tables
+    img = torch.randn((4, 64, 64), device="cuda")
+    kw = dict(img_shape=[64, 64], img_space=[0.7, 0.7], proj_shape=[90, 96], channel_space=1.3,
+              orbit=math.pi / 90)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    sinos = [torch.randn((n, 90, ns), device="cuda") for n, ns in ((4, 96), (16, 960), (3, 2000))]
+    outs = [torch.empty((len(s), 64, 64), device="cuda") for s in sinos]
+
+    def bp(k, stream):  # no allocation but the operator's own
+        n, na, ns = sinos[k].shape
+        p = FanBackprojection2DParam(ns, na, 1.3, 2 * math.pi / na, 0.0, 0.0, 64, 64, 0.7, 0.7,
+                                     0.0, 0.0, 595.0, 1085.6)
+        tabs = device_tables("fan", p, img.device)
+        _lib.call("ctr_fan_bp", C.byref(p.ctr()), 0, C.c_void_p(sinos[k].data_ptr()),
+                  C.c_void_p(outs[k].data_ptr()), n, *(C.c_void_p(t.data_ptr()) for t in tabs),
+                  p.scale, C.c_void_p(stream.cuda_stream))
+
+    want = F.parallel_projection_2d(img, **kw) * 2
+    for k in range(2):  # kept blocks, last used on two streams; the third size has none
+        bp(k, streams[0])
+        bp(k, streams[1])
+    bp(2, streams[0])
+    torch.cuda.synchronize()
+    F.release_workspace()
+    for k in range(2):
+        bp(k, streams[0])
+    images = [o.clone() for o in outs]
+    torch.cuda.synchronize()
+    go, done, errors = threading.Event(), threading.Event(), []
+
+    def work():
+        go.wait(60)
+        try:
+            for k in (0, 1, 2, 0, 1):
+                bp(k, streams[2])
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+        done.set()
+
+    t = threading.Thread(target=work)
+    t.start()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = F.parallel_projection_2d(img, **kw)
+        go.set()
+        assert done.wait(60)
+        z = y * 2
+    t.join()
+    assert not errors
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, want)
+    assert all(torch.equal(a, b) for a, b in zip(images, outs))
