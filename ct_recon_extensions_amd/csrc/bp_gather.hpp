@@ -1,4 +1,4 @@
-// Gather-form exact transpose of the pixel-driven BP engine, for float32.
+// Gather-form transpose of the pixel-driven BP, for float32.
 //
 // The BP sums, for every pixel and view, w * lerp(proj[view], s) with
 // s = s(pixel, view) and the taps floor(s), floor(s)+1.  Its transpose
@@ -19,9 +19,10 @@
 // pi ix + qj iy + rr with L >= 0 exactly where s >= s* (Geo::boundary).  On
 // one image row the pixels with s in [i-eps, i+1+eps] are then the
 // intersection of two half-lines, computed per row from two linear bounds;
-// each candidate is evaluated with the forward kernel's own per-tile
-// anchors and FP32 pixel geometry (Geo::pixel), so the weights are those of
-// the forward.  The margin eps (1/32 channel) keeps every pixel of the
+// each candidate is evaluated with the forward's per-tile anchors and the engine
+// kernel's FP32 pixel geometry (Geo::pixel).  Those are the engine's bits, and the
+// stream kernel's (bp_stream.hpp, the default forward) up to the rounding of a
+// position and what its run polynomials leave out, about 1e-6 channel.  The margin eps (1/32 channel) keeps every pixel of the
 // support inside the candidate interval despite FP32 rounding of the bounds.
 //
 // Work layout (gfx950): a workgroup = 4 views (one wave each) x 64 channel

@@ -1,6 +1,11 @@
-// Per-(pixel tile, view) fan-beam geometry, the policy the BP engine uses
-// for bp_fan_2d and bp_fan_2d_angle; the forward kernel and its transpose
-// evaluate bit-identical channel positions and weights through it.
+// Per-(pixel tile, view) fan-beam geometry of bp_fan_2d and bp_fan_2d_angle: the
+// policy of the BP engine and of the gather transpose, which evaluate the same bits
+// pixel by pixel (FanGeo), and of the stream kernel, the default forward, which
+// takes runs of pixels from a polynomial (FanRun).  Stream and transpose share the
+// anchors; their positions differ by rounding and by what the polynomial leaves
+// out (fan_run_order: 1e-6 channel and 4e-7 of the weight at most), so the pair is
+// adjoint to about 1e-6, and a pixel that lies within that of the detector's end
+// may count in one and not in the other.
 //
 // For a pixel at (x, y) and source angle beta (source at
 // (-dso sin b, dso cos b)) the reference computes, in FP64
@@ -212,7 +217,11 @@ struct FanGeo {
 // into the lower ones by its least-squares fit over the run's eight pixels,
 //     d^3 ~ 9.25 d, d^4 ~ 12.786 d^2 - 18.56, d^5 ~ 15.833 d^3 - 46.75 d,
 // which leaves 1/4, 1/6.8 and 1/16 of it.  fan_run_order says which form, if
-// any, leaves less than the rounding of f and w.
+// any, leaves less than the rounding of f and w.  Against FP64 the BP of filtered
+// scans (210^2 to 1024^2, 1 to 30 slices) is 0.6e-7 to 3.6e-7 relative L2 off, the
+// engine kernel on the same data 0.9e-7 to 3.8e-7, and on none of them less; on
+// sinograms of one sign 16 slices are up to 1.13 times the engine's 2.4e-7 (chains
+// of 90 views against 64).
 template <bool LONG>
 struct FanRun : FanGeo<false> {
     using StreamAnchor = FanStreamAnchor;

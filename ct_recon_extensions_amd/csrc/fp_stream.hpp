@@ -15,7 +15,10 @@
 //    nx - 1; where a crossing falls within 1e-8 of a row the accumulation is
 //    replayed, elsewhere its rounding cannot matter).  Inside them the position
 //    is 32.32 fixed point: an add, an add with carry, and the fraction's
-//    conversion per sample, good to 2^-33 of a pixel a step;
+//    conversion per sample, good to 2^-33 of a pixel a step, restarted from FP64
+//    in each segment.  Noise images against FP64, relative L2: 2.0e-7 at 256^2,
+//    2.8e-7 at 512^2, 1.1e-6 at 8192^2 (positions accumulated in FP64 and one FP32
+//    sum a ray, as before: 3.7e-7, 5.3e-7, 1.5e-6);
 //  * rows on which all rays of the wave are inside run without any test; the
 //    columns of every chunk are computed 64 chunks at a time, one a lane.
 #pragma once

@@ -125,3 +125,29 @@ def test_float64_integer_positions_read_one_channel(n):
         np.testing.assert_array_equal(np.isfinite(out[b]), np.isfinite(want))
         ok = np.isfinite(want)
         assert rel_l2(out[b][ok], want[ok]) < 1e-12, b
+
+
+@pytest.mark.parametrize("fan", [True, False])
+@pytest.mark.parametrize("ns,offset_s", [(40, 0.0), (41, 11.0), (40, 0.25)])
+@pytest.mark.parametrize("n", [1, 4, 16])
+def test_pair_is_adjoint_on_truncated_detectors(fan, ns, offset_s, n):
+    """Forward (runs of pixels) and transpose (pixel by pixel) where many tiles reach
+    past the detector.  1e-6 for rounding, and one pixel-view that lies within rounding
+    of the detector's end may count in one only: 1 / (pixels sqrt(views)) of the norms."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import ct_recon_extensions_amd as F
+    side, na = 96, 60
+    kw = dict(img_shape=[side, side], img_space=[0.7, 0.7], proj_shape=[na, ns], channel_space=1.3,
+              img_offset=[0.3, -0.7], channel_offset=offset_s, orbit_start=0.1,
+              orbit=(2 if fan else 1) * math.pi / na)
+    if fan:
+        kw.update(dso=595.0, dsd=1085.6)
+        A, At = F.fan_backprojection_2d, F.fan_backprojection_2d_grad
+    else:
+        A, At = F.parallel_backprojection_2d, F.parallel_backprojection_2d_grad
+    x = torch.from_numpy(randn(1680, (n, na, ns))).cuda()
+    y = torch.from_numpy(randn(1681, (n, side, side))).cuda()
+    ax, aty = A(x, **kw).double(), At(y, **kw).double()
+    gap = abs((ax * y).sum() - (x * aty).sum()) / (ax.norm() * y.double().norm())
+    assert gap < 1e-6 + 1.0 / (side * side * math.sqrt(na))
