@@ -562,6 +562,40 @@ inline bool stream_applies(int lmax, long long na, long long ns)
     return stream_reaches(lmax, na, ns, 4) && na <= 8 * 2 * kStreamChain;
 }
 
+// Whether the stream kernels are the faster for n slices of nx x ny pixels.  A tile's
+// 8 or 16 waves have to be worth their sums at the end, and the interleaved copy its
+// two passes over the sinogram; the engine kernel has neither (4 waves a tile, no copy),
+// and the fewer views, the more both weigh.  It pads a batch to whole groups of `most`
+// (16; the FP transpose 8), 8, 4 or 2 slices, and on a small image it leaves the chip
+// half empty.  Measured on fan, parallel and FP-transpose calls of 32^2 to 1024^2 with 8
+// to 720 views and 1 to 32 slices, engine -> stream in us:
+//  * one slice from 56 views on (fan 512^2: 30 views 11 -> 14, 60 views 17 -> 16);
+//  * 2 or 3 from 144 (512^2, 2 slices: 90 views 26 -> 30, 180 views 47 -> 41);
+//  * 4 or more from 176 on images of up to 256 tiles (256^2, 8 slices: 90 views 24 ->
+//    26, 180 views 44 -> 31), on larger ones from 144 for a batch that the engine pads
+//    (512^2, 5 slices: 90 views 53 -> 49) and from 208 for one that it does not (512^2,
+//    8 slices: 120 views 46 -> 56, 240 views 87 -> 82);
+//  * a batch of 16s and a rest is two or three launches here: from 208 views on, 240 on
+//    images of up to 512 tiles, 480 for the FP transpose there (24 slices of 320^2, 320
+//    views 179 -> 208);
+//  * where the anchors of many views keep groups of 16 out of the LDS (spans of 64
+//    channels, 1536 views), two groups of 8 take longer than one of the engine's 16
+//    (400^2, 16 slices: 879 and 983 us).
+inline bool stream_pays(int n, int nx, int ny, int na, int lmax, int most)
+{
+    const long long tiles = static_cast<long long>(div_up(nx, kStreamTile)) * div_up(ny, kStreamTile);
+    const int group = std::min(most, n >= 16 ? 16 : n >= 8 ? 8 : n >= 4 ? 4 : n >= 2 ? 2 : 1);
+    int least = n == 1         ? 56
+                : n < 4        ? 144
+                : tiles <= 256 ? 176
+                : n % group    ? 144
+                               : 208;
+    if (n > 16 && n % 16) least = tiles > 512 ? 208 : most == 8 ? 480 : 240;
+    if (na < least) return false;
+    const bool sixteens = most == 16 && n >= 16 && (n % 16 == 0 || n % 16 > 8);
+    return !sixteens || stream_fits<16, 4>(na, (lmax + 15) / 16 * 16);
+}
+
 // A batch of n sinograms proj, in groups of 16, 8, 4 (2, 1) slices.  A group
 // costs about 326, 199, 141, 110, 83 us of 512^2 pixels and 720 views, empty
 // slices included: 10 to 15 slices are one group of 16 (8 + 4: 340), 5 to 7 one

@@ -475,7 +475,8 @@ int fan_bp_f32(const ctr_geom& g, const float* proj, float* img, int nbatch, con
     }
     const FanTables T{xpos, ypos, sc};
     const int order = cfg.tile == 0 && cfg.vchunk == 0 && cfg.nb == 0 && !exact &&
-                              stream_applies(lmax, g.na, g.ns)
+                              stream_applies(lmax, g.na, g.ns) &&
+                              stream_pays(nbatch, P.nx, P.ny, P.na, lmax, 16)
                           ? fan_run_order(g)
                           : 0;
     if (order) {

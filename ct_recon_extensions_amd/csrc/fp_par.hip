@@ -525,7 +525,7 @@ int fpt_typed(const ctr_geom& g, const T* proj, T* img, int nbatch, const double
             int rc = CTR_OK;
             FpProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
                         static_cast<int>(g.ny), nbatch, g.dx, g.dy};
-            if (stream_applies(48, g.na, g.ns)) {
+            if (stream_applies(48, g.na, g.ns) && stream_pays(nbatch, P.nx, P.ny, P.na, 48, 8)) {
                 StreamLaunch<FptGeo> S{};
                 S.P = FptProblem{P.ns, P.na, P.nx, P.ny};
                 S.scale = 1.0;

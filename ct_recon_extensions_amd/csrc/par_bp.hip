@@ -285,7 +285,8 @@ int par_bp(const ctr_geom& g, int dtype, const void* proj, void* img, int nbatch
     const ParTables T{xcos, ysin};
     L.proj = static_cast<const float*>(proj);
     L.img = static_cast<float*>(img);
-    if (stream_applies(L.lmax, g.na, g.ns)) {
+    if (stream_applies(L.lmax, g.na, g.ns) &&
+        stream_pays(nbatch, L.P.nx, L.P.ny, L.P.na, L.lmax, 16)) {
         StreamLaunch<ParGeo> S{};
         S.P = L.P;
         S.scale = g.orbit;

@@ -1,7 +1,7 @@
-"""Backprojection where a view's span starts before its sinogram does: one tile, one
-view a wave, the first view's first tap on channel 0.  The span then starts at
-channel -1, four (or two) channels a lane, and the channels from 0 on still count.
-Against the oracle, at the suite's 1e-5 relative L2."""
+"""Backprojection at the edges of sinograms and detectors, against the oracle at the
+suite's 1e-5 relative L2.  Where the first view's first tap is channel 0, its span
+starts at channel -1, before the sinogram, four (or two) channels a lane, and the
+channels from 0 on still count."""
 import math
 
 import pytest
@@ -20,7 +20,8 @@ def test_first_channels_of_the_first_view(n, first):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     import ct_recon_extensions_amd as F
-    ns, na, start = 48, 8, 0.1
+    # the tile reaches farthest in view 0, so all views are inside the detector
+    ns, na, start = 48, 200, math.pi / 4
     reach = 7.5 * (math.cos(start) + math.sin(start))  # of the tile in view 0, both ways
     g = dict(nx=16, ny=16, na=na, ns=ns, dx=1.0, dy=1.0, ds=1.0, offset_x=0.0, offset_y=0.0,
              offset_s=first + reach - (ns - 1) / 2, orbit_start=start, orbit=math.pi / na)
@@ -46,22 +47,28 @@ def test_first_channels_of_the_first_fan_view(kind):
     import ct_recon_extensions_amd as F
     from ct_recon_extensions_amd import ragged
     from ct_recon_extensions_amd.geometry import FanBackprojection2DAngleParam
-    ns, na, n, dx, ds, dso, dsd = 64, 4, 16, 0.7, 1.3, 595.0, 1085.6
-    # the largest channel distance of a pixel from the centre in the view at angle 0,
-    # found on the pixels themselves
+    ns, na, n, dx, ds, dso, dsd = 64, 200, 16, 0.7, 1.3, 595.0, 1085.6
+    # the first view is the one in which the tile reaches farthest, so all views are
+    # inside the detector
     x = (np.arange(n) - (n - 1) / 2) * dx
-    s = np.arctan2(x[None, :], dso - x[::-1, None]) * dsd / ds
-    off = 0.6 - s.min() - (ns - 1) / 2
-    angles = 2 * math.pi / na * np.arange(na)
+    y = x[::-1, None]
+
+    def first(b):
+        r, d = x * np.cos(b) + y * np.sin(b), dso + x * np.sin(b) - y * np.cos(b)
+        return (np.arctan2(r, d) * dsd / ds).min()
+
+    start = min(2 * math.pi / na * np.arange(na), key=first)
+    off = 0.6 - first(start) - (ns - 1) / 2
+    angles = start + 2 * math.pi / na * np.arange(na)
     og = O.geom(nx=n, ny=n, na=na, ns=ns, dx=dx, dy=dx, ds=ds, offset_x=0.0, offset_y=0.0,
-                offset_s=off, orbit_start=0.0, orbit=2 * math.pi / na, dso=dso, dsd=dsd)
+                offset_s=off, orbit_start=start, orbit=2 * math.pi / na, dso=dso, dsd=dsd)
     proj = randn(1650, (na, ns))
     proj[0, :4] *= 10.0
     want = O.fan_bp(og, proj, O.fan_prep(og))
     if kind == "fan":
         out = F.fan_backprojection_2d(
             torch.from_numpy(proj)[None].cuda(), img_shape=[n, n], img_space=[dx, dx],
-            proj_shape=[na, ns], channel_space=ds, channel_offset=off, orbit_start=0.0,
+            proj_shape=[na, ns], channel_space=ds, channel_offset=off, orbit_start=start,
             orbit=2 * math.pi / na, dso=dso, dsd=dsd)[0]
     else:
         p = FanBackprojection2DAngleParam(ns, na, ds, off, n, n, dx, dx, 0.0, 0.0, dso, dsd)
@@ -137,7 +144,7 @@ def test_pair_is_adjoint_on_truncated_detectors(fan, ns, offset_s, n):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     import ct_recon_extensions_amd as F
-    side, na = 96, 60
+    side, na = 96, 180
     kw = dict(img_shape=[side, side], img_space=[0.7, 0.7], proj_shape=[na, ns], channel_space=1.3,
               img_offset=[0.3, -0.7], channel_offset=offset_s, orbit_start=0.1,
               orbit=(2 if fan else 1) * math.pi / na)

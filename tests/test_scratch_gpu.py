@@ -40,7 +40,7 @@ import ct_recon_extensions_amd as F
 from ct_recon_extensions_amd import _lib
 _lib.load()
 torch.manual_seed(3)
-na, ns, side = 90, 96, 70
+na, ns, side = 240, 96, 70
 kw = dict(img_shape=[side, side], img_space=[0.7, 0.7], proj_shape=[na, ns], channel_space=1.3,
           orbit=math.pi / na)
 fan = dict(kw, orbit=2 * math.pi / na, dso=595.0, dsd=1085.6)
@@ -121,7 +121,7 @@ def test_calls_beside_another_threads_capture():
     kw = dict(img_shape=[64, 64], img_space=[0.7, 0.7], proj_shape=[90, 96], channel_space=1.3,
               orbit=math.pi / 90)
     streams = [torch.cuda.Stream() for _ in range(3)]
-    sinos = [torch.randn((n, 90, ns), device="cuda") for n, ns in ((4, 96), (16, 960), (3, 2000))]
+    sinos = [torch.randn((n, 240, ns), device="cuda") for n, ns in ((4, 96), (16, 960), (3, 2000))]
     outs = [torch.empty((len(s), 64, 64), device="cuda") for s in sinos]
 
     def bp(k, stream):  # no allocation but the operator's own
