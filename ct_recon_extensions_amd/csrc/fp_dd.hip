@@ -513,14 +513,23 @@ __global__ __launch_bounds__(256) void fp_dd_grad_planes_kernel(
             img[(static_cast<size_t>(b0 + k) * P.ny + iy) * P.nx + ix] = static_cast<float>(sum[k]);
 }
 
+// Whether 1 to 4 slices that 8s leave over go along as one more, padded group of 8:
+// a launch of their own takes as long as the whole one where that does not fill the
+// chip (blocks: workgroups of a group; FP of 9 slices of 256^2, 60 views: 396 us in
+// two launches, 282 in one; 9 of 512^2, 360 views, 1068 and 1150).
+bool dd_padded(int nbatch, long long blocks)
+{
+    return nbatch > 8 && nbatch % 8 >= 1 && nbatch % 8 <= 4 && blocks * div_up(nbatch, 8) < 800;
+}
+
 // Slices in groups of 8, 4 and 1 (2 and 3 left over are one group of 4).
 template <typename F>
-int dd_groups(int nbatch, F&& launch)
+int dd_groups(int nbatch, bool padded, F&& launch)
 {
     for (int b0 = 0; b0 < nbatch;) {
         const int left = nbatch - b0;
         const int nb = left >= 5 ? 8 : left >= 2 ? 4 : 1;
-        const int take = nb == 8 && left >= 8 ? left / 8 * 8 : std::min(left, nb);
+        const int take = padded ? left : nb == 8 && left >= 8 ? left / 8 * 8 : std::min(left, nb);
         const int rc = launch(b0, take, nb);
         if (rc) return rc;
         b0 += take;
@@ -534,7 +543,9 @@ int fp_dd_f32_part(const ctr_geom& g, const float* img, float* proj, int nbatch,
     DdProblem P{static_cast<int>(g.ns), static_cast<int>(g.na), static_cast<int>(g.nx),
                 static_cast<int>(g.ny), nbatch, g.dx, g.dy};
     const size_t slice = static_cast<size_t>(g.nx) * g.ny;
-    const bool single = nbatch % 8 == 1;  // a last slice alone
+    const bool padded = dd_padded(
+        nbatch, static_cast<long long>(div_up(g.ns, 64)) * div_up(g.na, kDdViews));
+    const bool single = nbatch % 8 == 1 && !padded;  // a last slice alone
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
     float* ws = nullptr;
     const int e = ws_part(reinterpret_cast<void**>(&ws),
@@ -550,7 +561,7 @@ int fp_dd_f32_part(const ctr_geom& g, const float* img, float* proj, int nbatch,
                            one + slice, P.ny, P.nx, 1);
     int rc = check_launch("dd_cells_kernel");
     if (rc == CTR_OK)
-        rc = dd_groups(nbatch, [&](int b0, int take, int nb) {
+        rc = dd_groups(nbatch, padded, [&](int b0, int take, int nb) {
             P.nbatch = take;
             float* out = proj + static_cast<size_t>(b0) * g.na * g.ns;
             const dim3 grid(div_up(g.ns, 64), div_up(g.na, kDdViews), div_up(take, nb));
@@ -585,8 +596,10 @@ int fp_dd_grad_f32_part(const ctr_geom& g, const float* proj, float* img, int nb
                            proj, ws, static_cast<unsigned int>(sino), nbatch);
     }
     int rc = check_launch("interleave_kernel");
+    const bool padded =
+        dd_padded(nbatch, static_cast<long long>(div_up(g.nx, 64)) * div_up(g.ny, 4));
     if (rc == CTR_OK)
-        rc = dd_groups(nbatch, [&](int b0, int take, int nb) {
+        rc = dd_groups(nbatch, padded, [&](int b0, int take, int nb) {
             P.nbatch = take;
             float* out = img + static_cast<size_t>(b0) * g.nx * g.ny;
             const dim3 grid(div_up(g.nx, 64), div_up(g.ny, 4), div_up(take, nb));
@@ -703,9 +716,18 @@ int fp_dd_grad(const ctr_geom& g, int dtype, const void* proj, void* img, int nb
 {
     CTR_REQUIRE(g.ns >= 1 && g.na >= 1 && g.nx >= 1 && g.ny >= 1, CTR_ERR_ARG,
                 "distance-driven FP gradient: sizes must be positive");
-    if (dtype == CTR_F32)
+    if (dtype == CTR_F32) {
+        // The kernel without interleaved planes (the same bits): where a few views are not
+        // worth the copy (2 slices of 128^2: 12 views 12 -> 17 us with it, 60 views 51 ->
+        // 47; 512^2, 4 slices, 12 views 24 and 24), and sinograms past its 32-bit positions.
+        const long long sino = static_cast<long long>(g.na) * g.ns;
+        const long long pixels = static_cast<long long>(g.nx) * g.ny;
+        if (nbatch > 1 && ((g.na <= 40 && pixels <= (1 << 17)) || sino >= (1LL << 31)))
+            return fp_dd_grad_typed(g, static_cast<const float*>(proj), static_cast<float*>(img),
+                                    nbatch, w, pos, usex, pos_stride, st);
         return fp_dd_grad_f32(g, static_cast<const float*>(proj), static_cast<float*>(img), nbatch,
                               w, pos, usex, static_cast<int>(pos_stride), st);
+    }
     return fp_dd_grad_typed(g, static_cast<const double*>(proj), static_cast<double*>(img),
                             nbatch, w, pos, usex, pos_stride, st);
 }

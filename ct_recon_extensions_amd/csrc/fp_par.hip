@@ -334,8 +334,9 @@ int fp_stream_shape(const ctr_geom& g)
     return -1;
 }
 
-// waves: of the groups of four; waves1: of a last slice alone.
-int fp_stream_part(const ctr_geom& g, int shape, int waves, int waves1, const float* img,
+// waves: of the groups of four; waves1: of a last slice alone; padded: that slice is a
+// group of four (the same bits).
+int fp_stream_part(const ctr_geom& g, int shape, int waves, int waves1, bool padded, const float* img,
                    float* proj, int nbatch, const double* sc, const double* bo, const int* usex,
                    hipStream_t st)
 {
@@ -348,7 +349,7 @@ int fp_stream_part(const ctr_geom& g, int shape, int waves, int waves1, const fl
     L.usex = usex;
     const size_t slice = static_cast<size_t>(g.nx) * g.ny;
     const int np = nbatch > 1 ? div_up(nbatch, 4) : 0;
-    const bool single = nbatch % 4 == 1;  // the last slice alone
+    const bool single = nbatch % 4 == 1 && !(padded && nbatch > 1);  // the last slice alone
     float* ws = nullptr;
     const int e = ws_part(reinterpret_cast<void**>(&ws),
                           (8 * np + (single ? 1 : 0)) * slice * sizeof(float), st);
@@ -369,7 +370,7 @@ int fp_stream_part(const ctr_geom& g, int shape, int waves, int waves1, const fl
         L.rows = rows;
         L.cols = cols;
         if (left >= 2) {
-            take = left % 4 == 1 ? left - 1 : left;
+            take = single ? left - 1 : left;
             rc = launch_fp_stream<4>(shape, L, take, waves, st);
         } else {
             L.rows = img;                   // indexed by slice
@@ -386,18 +387,25 @@ int fp_stream(const ctr_geom& g, int shape, const float* img, float* proj, int n
               const double* sc, const double* bo, const int* usex, hipStream_t st)
 {
     const size_t slice = static_cast<size_t>(g.nx) * g.ny, sino = static_cast<size_t>(g.na) * g.ns;
-    // of the whole call, whatever its parts are
-    const int four = nbatch % 4 == 1 ? nbatch - 1 : nbatch;  // slices in groups of four
+    // of the whole call, whatever its parts are.  A last slice alone is two more
+    // launches, which a small scan does not hide: there it is a padded group (5 slices
+    // of 32^2: 26 us alone, 17 padded)
+    const long long blocks = static_cast<long long>(div_up(g.ns, 64)) *
+                             div_up(g.na, shape < 2 ? 4 : 1) * div_up(nbatch, 4);
+    const bool padded = blocks < 512;
+    const int four = nbatch % 4 == 1 && !padded ? nbatch - 1 : nbatch;  // in groups of four
     const int waves = fp_stream_waves(g, shape, div_up(four, 4));
     const int waves1 = fp_stream_waves(g, shape, 1);
     const auto part = [&](int b, int count, int w1) {
-        return fp_stream_part(g, shape, waves, w1, img + b * slice, proj + b * sino, count, sc, bo,
-                              usex, st);
+        return fp_stream_part(g, shape, waves, w1, padded, img + b * slice, proj + b * sino, count,
+                              sc, bo, usex, st);
     };
     return in_parts(
         nbatch, 2 * slice * sizeof(float), [&](int b, int count) { return part(b, count, waves1); },
         [&](int b, int count) {
-            return one_by_one(b, count, [&](int i) { return part(i, 1, i < four ? waves : waves1); });
+            return one_by_one(b, count, [&](int i) {
+                return part(i, 1, nbatch > 1 && i < four ? waves : waves1);
+            });
         });
 }
 
