@@ -132,7 +132,8 @@ __device__ __forceinline__ StageLane stage_lane(int pitch, int lane)
 // 4 bytes a lane, the slices apart, the DMAs of 4-slice groups cost as much as
 // the sums (the 4-slice BP of 512^2, 720 views: 227 us against 150).
 // RAW (calls that must not or cannot allocate) stages the sinograms as they are, 4
-// bytes a lane: the same spans, hence the same sums.
+// bytes a lane: the same spans, hence the same sums (FP transpose of 512^2, 720 views,
+// engine -> RAW -> interleaved: 8 slices 249, 222, 206 us, 16 slices 453, 352, 335).
 // Off the detector: without EDGE every tap is inside, and what the span holds
 // past the row is not read (past the last row's end a 16-byte load still brings
 // the channels before the end; stream_tile keeps spans before the first row's
@@ -150,29 +151,38 @@ __device__ __forceinline__ void stream_stage(const StreamLaunch<Geo>& L, const S
     const unsigned int bytes = static_cast<unsigned int>(P.na) * row_bytes;  // of a slice group
     const size_t group = static_cast<size_t>(P.na) * P.ns * S::kIl;
     if constexpr (RAW && NB > 1) {
+        // lane -> slice lane % kIl, channel lane / kIl: its offset in the group's first
+        // 64 words is fixed for the tile.  Without EDGE a channel before or past the row
+        // reads a neighbour (or zero) and is no tap.
         const unsigned int slice_bytes = static_cast<unsigned int>(P.na) * P.ns * 4u;
+        const int lane_ch = lane / S::kIl, words = L.pitch * S::kIl;
+        const unsigned int lane_off =
+            (lane % S::kIl) * slice_bytes + static_cast<unsigned int>(lane_ch) * 4u;
 #pragma unroll 1
-        for (int e = 0; e < nv * S::kGroups; ++e) {
-            const int t = e / S::kGroups, g = e - t * S::kGroups;
-            const int is0 = anchors[vc + t].is0;
-            const unsigned int row = static_cast<unsigned int>(va + vc + t) * P.ns * 4u;
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<float*>(src + g * group), 0,
-                static_cast<unsigned int>(max(0, min(S::kIl, nb - S::kIl * g))) * slice_bytes,
-                0x00020000);
+        for (int t = 0; t < nv; ++t) {
+            const int is0 = uniform_i(anchors[vc + t].is0);
+            const unsigned int at =
+                lane_off + static_cast<unsigned int>((va + vc + t) * P.ns + is0) * 4u;
 #pragma unroll 1
-            for (int w0 = 0; w0 < L.pitch * S::kIl; w0 += 64) {
-                const int w = w0 + lane, ch = is0 + w / S::kIl;
-                const unsigned int voff =
-                    static_cast<unsigned int>(ch) < static_cast<unsigned int>(P.ns)
-                        ? (w % S::kIl) * slice_bytes + row + static_cast<unsigned int>(ch) * 4u
-                        : 0x80000000u;
-                if (w < L.pitch * S::kIl)
+            for (int w0 = 0; w0 < words; w0 += 64) {
+                unsigned int voff = at + w0 / S::kIl * 4;
+                if constexpr (EDGE)
+                    if (static_cast<unsigned int>(is0 + lane_ch + w0 / S::kIl) >=
+                        static_cast<unsigned int>(P.ns))
+                        voff = 0x80000000u;
+                if (w0 + lane >= words) continue;
+#pragma unroll
+                for (int g = 0; g < S::kGroups; ++g) {
+                    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                        const_cast<float*>(src + g * group), 0,
+                        static_cast<unsigned int>(max(0, min(S::kIl, nb - S::kIl * g))) * slice_bytes,
+                        0x00020000);
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(
                         rs,
                         (__attribute__((address_space(3))) void*)(
                             buf + (t * NB + g * S::kIl) * L.pitch + w0),
                         4, voff, 0, 0, 0);
+                }
             }
         }
     } else if constexpr (EDGE && S::kIl < 4) {
