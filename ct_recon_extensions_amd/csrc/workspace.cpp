@@ -63,12 +63,20 @@ bool capturing(hipStream_t st)
 
 // Another thread may be capturing a graph, which (in the global mode, PyTorch's
 // default) calls like hipEventQuery and hipMallocAsync from any thread would
-// invalidate; none of those made here touches a captured stream.
+// invalidate; none of those made here touches a captured stream.  Waiting for an
+// event and recording one need no such cover, so a call that finds its own stream's
+// block pays nothing for it.
 struct RelaxedCapture {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
+
+hipError_t event_passed(hipEvent_t e)
+{
+    const RelaxedCapture relaxed;
+    return hipEventQuery(e);
+}
 
 }  // namespace
 
@@ -80,7 +88,6 @@ hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     const size_t want = block_size(bytes);
-    const RelaxedCapture relaxed;
     try {
         std::lock_guard<std::mutex> lock(g_mu);
         Device& D = g_devices[dev];
@@ -88,7 +95,7 @@ hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
         for (size_t i = D.free.size(); i-- > 0;) {
             Block b = D.free[i];
             if (b.bytes < bytes || b.bytes > 2 * want) continue;
-            if (b.st != st && hipEventQuery(b.done) != hipSuccess) {
+            if (b.st != st && event_passed(b.done) != hipSuccess) {
                 (void)hipGetLastError();  // not ready
                 continue;
             }
@@ -101,6 +108,7 @@ hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
             *p = b.p;
             return hipSuccess;
         }
+        const RelaxedCapture relaxed;
         Block b{nullptr, want, nullptr, st};
         e = hipEventCreateWithFlags(&b.done, hipEventDisableTiming);
         if (e != hipSuccess) return e;
@@ -136,12 +144,12 @@ hipError_t ws_free(void* p, hipStream_t st)
         std::lock_guard<std::mutex> lock(g_mu);
         const auto it = g_used.find(p);
         if (it == g_used.end()) return hipFreeAsync(p, st);  // a captured allocation
-        const RelaxedCapture relaxed;
         Block b = it->second;
         g_used.erase(it);
         b.st = st;
         e = hipEventRecord(b.done, st);
         if (e != hipSuccess) {
+            const RelaxedCapture relaxed;
             (void)hipEventDestroy(b.done);
             const hipError_t f = hipFreeAsync(p, st);
             return f != hipSuccess ? f : e;
@@ -150,6 +158,7 @@ hipError_t ws_free(void* p, hipStream_t st)
         D.free.push_back(b);
         D.free_bytes += b.bytes;
         while (D.free_bytes > kKeep || D.free.size() > kBlocks) {
+            const RelaxedCapture relaxed;
             const Block old = D.free.front();
             D.free.pop_front();
             D.free_bytes -= old.bytes;
