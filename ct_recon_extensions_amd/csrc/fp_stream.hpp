@@ -127,20 +127,32 @@ __device__ __forceinline__ int wave_min(int x)
     return uniform_i(x);
 }
 
+// A chunk's column count, with kFpNarrow where a single slice's lanes move one column
+// each: four of a lane would cross the row's end.
+constexpr int kFpNarrow = 1 << 16;
+
+template <int IL>
+__device__ __forceinline__ int fp_columns(const FpSpan& c, int rowlen)
+{
+    const bool narrow = IL == 1 && c.first + ((c.cols + 3) & ~3) > rowlen && ((rowlen - c.first) & 3);
+    return c.cols + (narrow ? kFpNarrow : 0);
+}
+
 // DMA of the chunk's rows k0 .. k0 + kRows - 1, columns cm .. cm + cols - 1, of
 // every plane; columns past the row (the last column's right tap is one) and rows
 // past the image read as zero.
 template <int NB, int SPAN>
 __device__ __forceinline__ void fp_stage(const float* src, size_t plane, int nsteps, int rowlen,
-                                         int k0, int cm, int cols, int planes, float* buf, int lane)
+                                         int k0, int cm, int cols_flag, int planes, float* buf,
+                                         int lane)
 {
     using S = FpShape<NB, SPAN>;
     const unsigned int row_bytes = static_cast<unsigned int>(rowlen) * S::kIl * 4u;
     const unsigned int bytes = static_cast<unsigned int>(nsteps) * row_bytes;
     // columns a lane moves: 16 bytes of them, or one where a lane's four would
-    // cross the row's end (single slices)
-    const int lane_cols =
-        S::kIl == 4 || (cm + ((cols + 3) & ~3) > rowlen && ((rowlen - cm) & 3)) ? 1 : 4;
+    // cross the row's end (single slices; flagged by fp_columns)
+    const int lane_cols = S::kIl == 4 || cols_flag >= kFpNarrow ? 1 : 4;
+    const int cols = cols_flag & (kFpNarrow - 1);
     for (int c = 0; c < cols; c += 64 * lane_cols) {
         const int lc = c + lane * lane_cols, col = cm + lc;
         if (lc >= S::kSpan) continue;
@@ -336,7 +348,7 @@ __global__ __launch_bounds__(512) void fp_stream_kernel(const FpStreamLaunch L)
         }
         const FpSpan c = fp_span(xmin, xmax, rowlen, S::kSpan);
         cm_l = c.first;
-        cols_l = h0 + lane < nchunks ? c.cols : 0;
+        cols_l = h0 + lane < nchunks ? fp_columns<S::kIl>(c, rowlen) : 0;
     };
     spans(0);
     int cm = uniform_i(cm_l);
