@@ -1,5 +1,6 @@
-"""The columns that a chunk of the ray-driven FP stages (csrc/fp_span.hpp, the
-kernel's own header compiled for the host) hold every tap that its rays read:
+"""The ray-driven FP's host and device arithmetic (csrc/fp_span.hpp, the kernel's own
+header compiled for the host): the rows of a ray are those that the reference's
+accumulation admits, and the columns that a chunk stages hold every tap its rays read:
 the fixed-point positions, row chunks, view groups and column bounds of
 fp_stream_kernel restated on the host, on the library's own tables.  A tap
 outside them is whatever LDS held before."""
@@ -8,6 +9,7 @@ import math
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 from ct_recon_extensions_amd import _lib
@@ -17,6 +19,29 @@ ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
 SOURCE = r"""
 #include "ct_recon_extensions_amd/csrc/fp_span.hpp"
 using namespace ctr;
+
+// rays of `count` whose rows differ from the accumulation's, or whose rows without a
+// test (fin to fout) are not all inside
+extern "C" long long wrong_rows(const double* x0, const double* off, const int* hi, const int* n,
+                                long long count)
+{
+    long long bad = 0;
+    for (long long i = 0; i < count; ++i) {
+        int kin, kout, fin, fout, a = 0, b = 0;
+        fp_ray_rows(x0[i], off[i], hi[i], n[i], kin, kout, fin, fout);
+        bool seen = false, free = true;
+        double x = x0[i];
+        for (int k = 0; k < n[i]; ++k, x += off[i]) {
+            const bool inside = x >= 0 && x <= hi[i];
+            if (inside && !seen) a = k;
+            if (inside) b = k + 1;
+            seen = seen || inside;
+            free = free && (inside || k < fin || k >= fout);
+        }
+        bad += a != kin || b != kout || !free;
+    }
+    return bad;
+}
 
 // taps read outside the staged columns (and how many were read); -1: no shape applies
 extern "C" long long outside(const ctr_geom* g, const double* bo, const int* usex, int rows,
@@ -74,15 +99,15 @@ extern "C" long long outside(const ctr_geom* g, const double* bo, const int* use
 
 
 @pytest.fixture(scope="module")
-def outside(tmp_path_factory):
+def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("spans")
     src, so = d / "spans.cpp", d / "spans.so"
     src.write_text(SOURCE)
-    subprocess.run(["g++", "-std=c++17", "-O2", "-shared", "-fPIC", f"-I{ROOT}", str(src), "-o",
+    subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-shared", "-fPIC", f"-I{ROOT}", str(src), "-o",
                     str(so)], check=True)
-    f = C.CDLL(str(so)).outside
-    f.restype = C.c_longlong
-    return f
+    lib = C.CDLL(str(so))
+    lib.outside.restype = lib.wrong_rows.restype = C.c_longlong
+    return lib
 
 
 # (nx, ny, channels, views, ds, offset, start): rays on the last column with 63, 64,
@@ -101,7 +126,7 @@ CASES = [
 
 @pytest.mark.parametrize("case", range(len(CASES)))
 @pytest.mark.parametrize("rows", [2, 4])
-def test_every_tap_is_staged(outside, case, rows):
+def test_every_tap_is_staged(lib, case, rows):
     nx, ny, ns, na, ds, offset, start = CASES[case]
     g = _lib.CtrGeom()
     g.nx, g.ny, g.ns, g.na, g.ds, g.dx, g.dy = nx, ny, ns, na, ds, 1.0, 1.0
@@ -110,6 +135,29 @@ def test_every_tap_is_staged(outside, case, rows):
     sc, bo, usex = (C.c_double * (2 * na))(), (C.c_double * (2 * na * ns))(), (C.c_int * na)()
     _lib.call("ctr_fp_tables", C.byref(g), sc, bo, usex)
     taps, widest = C.c_longlong(), C.c_int()
-    bad = outside(C.byref(g), bo, usex, rows, C.byref(taps), C.byref(widest))
+    bad = lib.outside(C.byref(g), bo, usex, rows, C.byref(taps), C.byref(widest))
     assert taps.value > 0 and widest.value > 0
     assert bad == 0, f"{bad} of {taps.value} taps"
+
+
+@pytest.mark.parametrize("decade", range(0, 15))
+@pytest.mark.parametrize("size", [300, 6000])
+def test_rows_are_those_of_the_accumulation(lib, decade, size):
+    """Steps from 2 columns a row down to 1e-14, of rays anywhere, on an end of the
+    image, crossing it exactly at a row, and near that."""
+    count = 40000 if size == 300 else 2500
+    rng = np.random.default_rng(2000 + decade)
+    n, hi = rng.integers(1, size, count), rng.integers(1, size, count)
+    off = np.minimum(10.0 ** (rng.uniform(0, 1, count) - decade), 2.0) * rng.choice([-1, 1], count)
+    off[rng.random(count) < 0.02] = 0.0
+    end, row = np.where(rng.random(count) < 0.5, 0, hi), rng.integers(0, n + 1)
+    kind = rng.integers(0, 5, count)
+    x0 = np.select(
+        [kind == 0, kind == 1, kind == 2, kind == 3],
+        [rng.uniform(-0.2, 1.2, count) * hi, end, end - off * row,
+         end - off * row + rng.uniform(-2e-13, 2e-13, count)],
+        end - off * rng.uniform(0, 1, count) * n + rng.uniform(-2e-8, 2e-8, count))
+    x0, off = np.ascontiguousarray(x0, np.float64), np.ascontiguousarray(off, np.float64)
+    hi, n = hi.astype(np.int32), n.astype(np.int32)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    assert lib.wrong_rows(p(x0), p(off), p(hi), p(n), C.c_longlong(count)) == 0
