@@ -77,7 +77,7 @@ struct ParGeo {
     using Problem = ParProblem;
     using Tables = ParTables;
     using Anchor = ParAnchor;
-    static constexpr bool kGatherFrac = true;
+    static constexpr bool kGatherFrac = false;  // the engine's positions
     __device__ static Anchor anchor(const Problem& P, const Tables& T, const TileFrame& F,
                                     int view, int ilo, int ihi, int jlo, int jhi)
     {
@@ -118,6 +118,11 @@ struct ParGeo {
         qj = P.ny > 1 ? (T.ysin[(P.ny - 1) * na + view] - ys0) / (P.ny - 1) : 0.0;
         rr = xc0 + ys0 - (s_star - P.cents) * P.ds;
     }
+};
+
+// The gather with the stream kernel's positions.
+struct ParStreamGeo : ParGeo {
+    static constexpr bool kGatherFrac = true;
 };
 
 // FP64 buffers: one thread per pixel, the reference's FP64 arithmetic.
@@ -230,6 +235,13 @@ int par_problem(const ctr_geom& g, int TW, int TH, ParProblem& P, int& lmax)
     return CTR_OK;
 }
 
+// Which forward kernel a call of nbatch slices takes (and which positions its
+// transpose, so that the pair stays adjoint to rounding).
+bool par_streams(const ParProblem& P, int lmax, int nbatch)
+{
+    return stream_applies(lmax, P.na, P.ns) && stream_pays(nbatch, P.nx, P.ny, P.na, lmax, 16);
+}
+
 template <int TW, int TH, int NB, int LROW>
 int launch_par_bp_l(BpLaunch<ParGeo> L, const ParTables& T, hipStream_t st)
 {
@@ -285,8 +297,7 @@ int par_bp(const ctr_geom& g, int dtype, const void* proj, void* img, int nbatch
     const ParTables T{xcos, ysin};
     L.proj = static_cast<const float*>(proj);
     L.img = static_cast<float*>(img);
-    if (stream_applies(L.lmax, g.na, g.ns) &&
-        stream_pays(nbatch, L.P.nx, L.P.ny, L.P.na, L.lmax, 16)) {
+    if (par_streams(L.P, L.lmax, nbatch)) {
         StreamLaunch<ParGeo> S{};
         S.P = L.P;
         S.scale = g.orbit;
@@ -321,8 +332,11 @@ int par_bpt(const ctr_geom& g, int dtype, const void* img, void* proj, int nbatc
         return check_launch("par_bpt_f64_gather_kernel");
     }
     const ParTables T{xcos, ysin};
-    return launch_bp_gather_t<ParGeo>(P, T, static_cast<const float*>(img),
-                                      static_cast<float*>(proj), nbatch, g.orbit, ws, st);
+    const auto* x = static_cast<const float*>(img);
+    auto* y = static_cast<float*>(proj);
+    return par_streams(P, lmax, nbatch)
+               ? launch_bp_gather_t<ParStreamGeo>(P, T, x, y, nbatch, g.orbit, ws, st)
+               : launch_bp_gather_t<ParGeo>(P, T, x, y, nbatch, g.orbit, ws, st);
 }
 
 }  // namespace ctr
