@@ -46,9 +46,10 @@ PEAK_VALU_SLOTS = CU * LANES * CLK  # FP32 VALU lane-issues per second (3.93e13)
 # Per slice: two FMAs into the accumulator = 2.
 FAN_GEOM_SLOTS = 24
 FAN_SLICE_SLOTS = 2
-# The forward BP evaluates that geometry once per run of 8 pixels, with its
-# derivatives (43 slots), and each pixel from the run's polynomial (3.5).
-FAN_RUN_SLOTS = 9
+# The forward BP evaluates that geometry once per run of pixels, with its
+# derivatives (43 slots), and each pixel from the run's polynomial (3.5): runs of 4
+# pixels in groups of 16 slices, of 8 in smaller ones and in ragged batches.
+FAN_RUN_SLOTS = {4: 43 / 4 + 3.5, 8: 43 / 8 + 3.5}
 # Per-slice model with no geometry sharing (atan2 + divide per pixel*view,
 # the textbook count for one slice at a time).
 UNBATCHED_FAN_SLOTS = 28
@@ -533,7 +534,7 @@ def bench_ragged(torch, reps):
             rb.pixel_views / (ms * 1e-3) * UNBATCHED_FAN_SLOTS / PEAK_VALU_SLOTS, 4),
         # one slice per problem: the geometry of every pixel*view is its own
         "roofline": _valu_roofline("ragged_fan_bp_kernel", rb.pixel_views,
-                                   FAN_RUN_SLOTS + FAN_SLICE_SLOTS, ms, "pixel*view"),
+                                   FAN_RUN_SLOTS[8] + FAN_SLICE_SLOTS, ms, "pixel*view"),
     }
     rb.close()
     return out
@@ -953,7 +954,7 @@ def main():
     bp_rate = pv_batch / (ms_bp * 1e-3)
     nb_group = 16
     groups = math.ceil(B / nb_group)
-    slots = pv_slice * FAN_RUN_SLOTS * groups + pv_batch * FAN_SLICE_SLOTS
+    slots = pv_slice * FAN_RUN_SLOTS[4] * groups + pv_batch * FAN_SLICE_SLOTS
     valu_achieved = slots / (ms_bp * 1e-3)
     hbm_bytes = B * 4 * (na * ns + n * n) + 16 * na + 8 * 2 * n
     hbm_achieved = hbm_bytes / (ms_bp * 1e-3) / 1e9
@@ -1043,7 +1044,7 @@ def main():
         "slices_per_s": round(B / (ms_step * 1e-3), 1),
         "kernels_ms": {"fan_filter": round(ms_filter, 4), "fan_bp": round(ms_bp, 4)},
         "roofline": {
-            "kernel": "fan_bp_kernel",
+            "kernel": "bp_stream_kernel<FanRun<false>, 16, 4> (with interleave_kernel<4>)",
             "bound": "valu",
             "achieved": round(valu_achieved / 1e12, 3),
             "peak": round(PEAK_VALU_SLOTS / 1e12, 3),
