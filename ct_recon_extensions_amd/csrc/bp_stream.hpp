@@ -131,9 +131,10 @@ __device__ __forceinline__ StageLane stage_lane(int pitch, int lane)
 // itself), so a lane moves 16 bytes: 4, 2 or 1 channels of 1, 2 or 4 slices.  With
 // 4 bytes a lane, the slices apart, the DMAs of 4-slice groups cost as much as
 // the sums (the 4-slice BP of 512^2, 720 views: 227 us against 150).
-// RAW (calls that must not or cannot allocate) stages the sinograms as they are, 4
-// bytes a lane: the same spans, hence the same sums (FP transpose of 512^2, 720 views,
-// engine -> RAW -> interleaved: 8 slices 249, 222, 206 us, 16 slices 453, 352, 335).
+// RAW (calls that must not or cannot allocate, or are captured) stages the sinograms
+// as they are, 4 bytes a lane: the same spans, hence the same sums (FP transpose of
+// 512^2, 720 views, engine -> RAW -> interleaved: 8 slices 249, 222, 206 us, 16 slices
+// 453, 352, 335).
 // Off the detector: without EDGE every tap is inside, and what the span holds
 // past the row is not read (past the last row's end a 16-byte load still brings
 // the channels before the end; stream_tile keeps spans before the first row's
@@ -669,9 +670,12 @@ int launch_stream_batch(StreamLaunch<Geo> L, const typename Geo::Tables& T, cons
         L.img = img + b * image;
         return launch_stream_part<Geo, decltype(raw)::value>(L, T, proj + b * sino, count, lmax, st);
     };
+    const auto raw = [&](int b, int count) { return part(std::true_type{}, b, count); };
+    const size_t bytes = sino * sizeof(float);
+    // a captured BP allocates nothing: no memory nodes in the graph
+    if (n > 1 && ws_capturing(st)) return in_parts(n, bytes, raw, raw);
     return in_parts(
-        n, sino * sizeof(float), [&](int b, int count) { return part(std::false_type{}, b, count); },
-        [&](int b, int count) { return part(std::true_type{}, b, count); });
+        n, bytes, [&](int b, int count) { return part(std::false_type{}, b, count); }, raw);
 }
 
 }  // namespace ctr

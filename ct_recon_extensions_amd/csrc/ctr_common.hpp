@@ -55,6 +55,8 @@ inline double cent_s(const ctr_geom& g) { return static_cast<double>(g.ns - 1) /
 // Device memory for the duration of a call, ordered on `st` (workspace.cpp).
 hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st);
 hipError_t ws_free(void* p, hipStream_t st);
+// Whether st is being captured: scratch is then a memory node of the graph.
+bool ws_capturing(hipStream_t st);
 
 // A batch in parts whose scratch (bytes a slice) stays within 1 GiB, at least 16
 // slices each: call(first, count).  A part whose scratch the device has no room for

@@ -51,16 +51,6 @@ size_t block_size(size_t bytes)
     return (bytes + step - 1) / step * step;
 }
 
-bool capturing(hipStream_t st)
-{
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return status != hipStreamCaptureStatusNone;
-}
-
 // Another thread may be capturing a graph, which (in the global mode, PyTorch's
 // default) calls like hipEventQuery and hipMallocAsync from any thread would
 // invalidate; none of those made here touches a captured stream.  Waiting for an
@@ -80,10 +70,21 @@ hipError_t event_passed(hipEvent_t e)
 
 }  // namespace
 
+bool ws_capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 hipError_t ws_alloc(void** p, size_t bytes, hipStream_t st)
 {
-    // a captured allocation belongs to the graph, which has memory of its own
-    if (capturing(st)) return hipMallocAsync(p, bytes, st);
+    // a captured allocation belongs to the graph, which has memory of its own (the
+    // forward BPs make none: bp_stream.hpp)
+    if (ws_capturing(st)) return hipMallocAsync(p, bytes, st);
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;

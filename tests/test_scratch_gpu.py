@@ -117,9 +117,9 @@ def test_calls_beside_another_threads_capture():
     import ct_recon_extensions_amd as F
     from ct_recon_extensions_amd import _lib
     from ct_recon_extensions_amd.geometry import FanBackprojection2DParam, device_tables
-    img = torch.randn((4, 64, 64), device="cuda")
+    x = torch.randn((1, 90, 96), device="cuda")
     kw = dict(img_shape=[64, 64], img_space=[0.7, 0.7], proj_shape=[90, 96], channel_space=1.3,
-              orbit=math.pi / 90)
+              orbit=math.pi / 90)  # one slice: the captured call itself takes no scratch
     streams = [torch.cuda.Stream() for _ in range(3)]
     sinos = [torch.randn((n, 240, ns), device="cuda") for n, ns in ((4, 96), (16, 960), (3, 2000))]
     outs = [torch.empty((len(s), 64, 64), device="cuda") for s in sinos]
@@ -128,12 +128,12 @@ def test_calls_beside_another_threads_capture():
         n, na, ns = sinos[k].shape
         p = FanBackprojection2DParam(ns, na, 1.3, 2 * math.pi / na, 0.0, 0.0, 64, 64, 0.7, 0.7,
                                      0.0, 0.0, 595.0, 1085.6)
-        tabs = device_tables("fan", p, img.device)
+        tabs = device_tables("fan", p, x.device)
         _lib.call("ctr_fan_bp", C.byref(p.ctr()), 0, C.c_void_p(sinos[k].data_ptr()),
                   C.c_void_p(outs[k].data_ptr()), n, *(C.c_void_p(t.data_ptr()) for t in tabs),
                   p.scale, C.c_void_p(stream.cuda_stream))
 
-    want = F.parallel_projection_2d(img, **kw) * 2
+    want = F.parallel_backprojection_2d(x, **kw) * 2
     for k in range(2):  # kept blocks, last used on two streams; the third size has none
         bp(k, streams[0])
         bp(k, streams[1])
@@ -159,7 +159,7 @@ def test_calls_beside_another_threads_capture():
     t.start()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        y = F.parallel_projection_2d(img, **kw)
+        y = F.parallel_backprojection_2d(x, **kw)
         go.set()
         assert done.wait(60)
         z = y * 2
