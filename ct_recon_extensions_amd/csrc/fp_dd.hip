@@ -516,7 +516,7 @@ __global__ __launch_bounds__(256) void fp_dd_grad_planes_kernel(
 // Whether 1 to 4 slices that 8s leave over go along as one more, padded group of 8:
 // a launch of their own takes as long as the whole one where that does not fill the
 // chip (blocks: workgroups of a group; FP of 9 slices of 256^2, 60 views: 396 us in
-// two launches, 282 in one; 9 of 512^2, 360 views, 1068 and 1150).
+// two launches, 273 in one; 9 of 512^2, 360 views, 1068 and 1150).
 bool dd_padded(int nbatch, long long blocks)
 {
     return nbatch > 8 && nbatch % 8 >= 1 && nbatch % 8 <= 4 && blocks * div_up(nbatch, 8) < 800;
